@@ -136,6 +136,8 @@ struct FamArgs {
     int mf;     // LDS capacity in members
     int maxpb;  // LDS capacity in PD-boundary entities per family (3D N.D cache)
     const int *flist = nullptr;  // families of the blocks (null: block f is family f)
+    double *fam_w = nullptr;     // MOM: weight mu_km omega V of every bond
+    double *fam_T = nullptr;     // MOM: the second-order rows of the inverse shape tensor [6][9] of every family
 };
 
 // normMatArea (pdsolve.cpp:2917-2967): area-weighted face normal matrix 3x6
@@ -263,7 +265,9 @@ __device__ inline void add_pdbe_term(const FamArgs &A, int p, const double *Cb, 
     }
 }
 
-template <int D>
+// MOM (3D): only the bond weights and the rows of the inverse shape tensor that the products by
+// moments read (hex.hpp); K and the strain weights stay as they are.
+template <int D, bool MOM = false>
 __global__ void __launch_bounds__(64) k_family(FamArgs A) {
     // no FMA contraction: the shape tensor of a one-sided family is ill-conditioned, and the
     // reference's arithmetic (separate multiply and add) must be followed to keep K to rounding
@@ -380,6 +384,41 @@ __global__ void __launch_bounds__(64) k_family(FamArgs A) {
         if (lane == 0) atomicOr(A.status, 1);
         return;
     }
+    // A x = b with the LU above
+    auto solve = [&](double (&b)[P], double (&s)[P]) {
+        // the LU swapped whole rows (multipliers included): permute b completely, then eliminate
+#pragma unroll
+        for (int kk = 0; kk < P; kk++) {
+            const int p = spiv[kk];
+#pragma unroll
+            for (int i = kk + 1; i < P; i++)
+                if (p == i) { double t = b[kk]; b[kk] = b[i]; b[i] = t; }
+        }
+#pragma unroll
+        for (int kk = 0; kk < P; kk++)
+#pragma unroll
+            for (int i = kk + 1; i < P; i++) b[i] = b[i] - sA[i * P + kk] * b[kk];
+#pragma unroll
+        for (int i = P - 1; i >= 0; i--) {
+            double t = b[i];
+#pragma unroll
+            for (int c = i + 1; c < P; c++) t = t - sA[i * P + c] * s[c];
+            s[i] = t / sA[i * P + i];
+        }
+    };
+    if constexpr (MOM) {
+        static_assert(D == 3, "products by moments are 3D");
+        for (int m = lane; m < n; m += 64) A.fam_w[off + m] = (double)A.bond[off + m] * som[m] * svm[m];
+        if (lane < P) {
+            double b[P], s[P];
+#pragma unroll
+            for (int i = 0; i < P; i++) b[i] = i == lane ? 1.0 : 0.0;
+            solve(b, s);
+#pragma unroll
+            for (int r = 0; r < 6; r++) A.fam_T[(size_t)f * 54 + r * 9 + lane] = s[3 + r];
+        }
+        return;
+    }
     const double cdv = A.fam_v[f];
     const double lam = A.lam, mu = A.mu;
     const int p0 = A.fp_off[f], p1 = A.fp_off[f + 1];
@@ -400,26 +439,8 @@ __global__ void __launch_bounds__(64) k_family(FamArgs A) {
             b[3] = x0 * x0; b[4] = x1 * x1; b[5] = x2 * x2;
             b[6] = x0 * x1; b[7] = x1 * x2; b[8] = x2 * x0;
         }
-        // the LU swapped whole rows (multipliers included): permute b completely, then eliminate
-#pragma unroll
-        for (int kk = 0; kk < P; kk++) {
-            const int p = spiv[kk];
-#pragma unroll
-            for (int i = kk + 1; i < P; i++)
-                if (p == i) { double t = b[kk]; b[kk] = b[i]; b[i] = t; }
-        }
-#pragma unroll
-        for (int kk = 0; kk < P; kk++)
-#pragma unroll
-            for (int i = kk + 1; i < P; i++) b[i] = b[i] - sA[i * P + kk] * b[kk];
         double s[P];
-#pragma unroll
-        for (int i = P - 1; i >= 0; i--) {
-            double t = b[i];
-#pragma unroll
-            for (int c = i + 1; c < P; c++) t = t - sA[i * P + c] * s[c];
-            s[i] = t / sA[i * P + i];
-        }
+        solve(b, s);
         const double om = som[m], vm = svm[m];
         const double mukm = (double)A.bond[off + m];
         double G[DD];
@@ -1093,6 +1114,27 @@ static int family_args(Ctx &c, int *status, FamArgs &A, size_t &lds, std::string
         err = "family too large for LDS (" + std::to_string(c.max_family) + " members)";
         return PDX_ERR_LIMIT;
     }
+    return PDX_OK;
+}
+
+// Bond weights and inverse shape tensors for the products by moments, for the bond states K was
+// assembled with
+int dev_family_moments(Ctx &c, std::string &err) {
+    if (c.mom_gen == c.K_gen) return PDX_OK;
+    FamArgs A;
+    size_t lds = 0;
+    if (int rc = family_args(c, c.asm_status, A, lds, err)) return rc;
+    if (!c.mom_w) {
+        const size_t nmem = c.host->fam_mem.size();
+        PDX_HIP(hipMalloc((void **)&c.mom_w, std::max<size_t>(nmem, 1) * sizeof(double)));
+        PDX_HIP(hipMalloc((void **)&c.mom_T, std::max<size_t>((size_t)c.nfam * 54, 1) * sizeof(double)));
+    }
+    A.fam_w = c.mom_w;
+    A.fam_T = c.mom_T;
+    PDX_HIP(hipFuncSetAttribute((const void *)k_family<3, true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    k_family<3, true><<<c.nfam, 64, lds, c.stream>>>(A);
+    PDX_HIP(hipGetLastError());
+    c.mom_gen = c.K_gen;
     return PDX_OK;
 }
 

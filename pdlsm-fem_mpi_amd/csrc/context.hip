@@ -23,6 +23,8 @@ int dev_newmark(Ctx &c, int nsteps, const pdx_solve_opts &o, std::vector<double>
                 std::string &err);
 int dev_explicit_state(Ctx &c, double *u_out, double *u_prev, std::string &err);
 int dev_max_eig(Ctx &c, int iters, double *lmax, std::string &err);
+int explicit_tune_seen(Ctx &c, int pi, std::string &err);
+void free_hex_tiles(Ctx &c);
 int stress_scratch_init(int device, std::string &err);
 int dev_node_stresses_noalloc(Ctx &c, const double *u_dev, double *sigma_dev, std::string &err);
 
@@ -473,9 +475,12 @@ void ctx_free(Ctx *c) {
     if (c->learned_Minv) hipFree(c->learned_Minv);
     if (c->gnn_keff) hipFree(c->gnn_keff);
     if (c->fam_c) hipFree(c->fam_c);
+    if (c->mom_w) hipFree(c->mom_w);
+    if (c->mom_T) hipFree(c->mom_T);
     if (c->Kown32) hipFree(c->Kown32);
     if (c->Kown64) hipFree(c->Kown64);
     if (c->stress_stage) hipFree(c->stress_stage);
+    free_hex_tiles(*c);
     free_two_level(*c);
     free_ilu0(*c);
     free_krylov_ws(*c);
@@ -959,8 +964,11 @@ int pdx_node_stresses_timed(pdx_ctx *pc, const double *u_all, double *ms) {
 int pdx_explicit_tuning(pdx_ctx *pc, int precision, int *lanes, int *nontemporal, int *xcd_order, int *row_soa,
                         int *col_classes, int *mirrored, int *alternating, int *form, float *ms) {
     if (!pc || (precision != PDX_FP64 && precision != PDX_FP32)) return fail(PDX_ERR_ARG, "bad argument");
-    const Ctx &c = *pc->c;
-    const int v = c.tune_explicit[precision];
+    Ctx &c = *pc->c;
+    std::string err;
+    hipSetDevice(c.device);
+    if (int rc = explicit_tune_seen(c, precision, err)) return fail(rc, err);
+    const int v = c.tune_explicit[precision] >= 0 ? c.tune_explicit[precision] : c.tune_seen[precision];
     const ExplicitForm f = v >= 0 ? kExplicitForms[v] : ExplicitForm{0, false, false, false, false, false, false, 0};
     if (lanes) *lanes = f.lanes;
     if (nontemporal) *nontemporal = f.nt;

@@ -166,6 +166,15 @@ struct Ctx {
     long long nlm_iters = 0;  // CG iterations of the mass solves so far
     double *dofs_tmp = nullptr;  // [nn*d] DOF values of the last stored step (stress input)
 
+    // node tiles of the products with hex8 elements without their K blocks (hex.hip)
+    void *hex = nullptr;
+    bool hex_tried = false;
+    // PD rows formed from the moments of their families (hex.hpp): bond weights [members] and the
+    // second-order rows of the inverse shape tensors [nfam * 54], for the K of generation mom_gen
+    double *mom_w = nullptr, *mom_T = nullptr;
+    long long mom_gen = -1;
+    int tune_seen[2] = {-1, -1};  // form the tuner found for a context that steps through the tiles
+
     // scratch for Krylov
     std::vector<DevBuf> scratch;
     double *red = nullptr;      // partial sums [RED_SLOTS * RED_PARTS]
@@ -212,6 +221,7 @@ int dev_assemble_K(Ctx &c, std::string &err);
 int dev_assemble_K_launch(Ctx &c, std::string &err);  // enqueue only
 int dev_assemble_K_finish(Ctx &c, std::string &err);  // wait, check the status word
 int dev_lumped_mass(Ctx &c, std::string &err);
+int dev_family_moments(Ctx &c, std::string &err);
 int dev_nbc_unit(Ctx &c, std::string &err);
 int dev_mass_on_K(Ctx &c, std::string &err);
 int dev_extract_csr(Ctx &c, const double *Kblk, double *Ku_dev);

@@ -1,0 +1,276 @@
+// Node tiles for the products with hex8 elements without their K blocks (hex.hpp): host set-up.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cmath>
+#include <cstring>
+#include <numeric>
+#include <vector>
+
+#include "hex.hpp"
+
+namespace pdx {
+
+namespace {
+
+// one tile under construction on the host
+struct HostTile {
+    int n_own = 0;
+    std::vector<int> node, ele, place;  // place: the elements in groups of HT_GROUP, -1 for an empty place
+    std::vector<unsigned short> conn;
+};
+
+void sort_along(std::vector<int> &v, size_t b, size_t e, const double *x, int axis) {
+    std::vector<std::pair<double, int>> k(e - b);
+    for (size_t i = b; i < e; i++) k[i - b] = {x[(size_t)v[i] * 3 + axis], v[i]};
+    std::sort(k.begin(), k.end());
+    for (size_t i = b; i < e; i++) v[i] = k[i - b].second;
+}
+
+// Nodes in slabs along x, the slabs in columns along y, each about `w` node spacings wide, the cuts
+// moved to the widest gap between neighbouring coordinates near the even position (so that a mesh
+// with layers is cut between layers); a column is then filled from below, node by node in z, until a
+// tile is full.
+void cut_even(std::vector<int> &v, size_t b, size_t e, const double *x, int axis, double width, std::vector<size_t> &cuts) {
+    sort_along(v, b, e, x, axis);
+    cuts.assign(1, b);
+    const size_t n = e - b;
+    const double ext = n ? x[(size_t)v[e - 1] * 3 + axis] - x[(size_t)v[b] * 3 + axis] : 0.0;
+    const size_t k = std::max<size_t>(1, (size_t)std::llround(ext / width));
+    for (size_t i = 1; i < k; i++) {
+        const size_t at = b + n * i / k, half = n / (4 * k) + 1;
+        size_t lo = at > cuts.back() + half ? at - half : cuts.back() + 1, best = at;
+        double gap = -1.0;
+        for (size_t q = lo; q < std::min(e, at + half); q++) {
+            const double d = x[(size_t)v[q] * 3 + axis] - x[(size_t)v[q - 1] * 3 + axis];
+            if (d > gap) {
+                gap = d;
+                best = q;
+            }
+        }
+        if (best > cuts.back()) cuts.push_back(best);
+    }
+    cuts.push_back(e);
+}
+
+// Elements into groups of HT_GROUP, in order, none beside another with the same node in the same
+// corner (two elements of a consistently numbered mesh never are)
+void place_elements(const Model &m, HostTile &t) {
+    std::vector<int> count;  // elements of each group
+    t.place.clear();
+    for (int e : t.ele) {
+        const int *ce = &m.econ[(size_t)e * 8];
+        size_t g = 0;
+        for (; g < count.size(); g++) {
+            if (count[g] == HT_GROUP) continue;
+            bool free = true;
+            for (int k = 0; k < count[g] && free; k++) {
+                const int *cf = &m.econ[(size_t)t.place[g * HT_GROUP + k] * 8];
+                for (int a = 0; a < 8; a++) free = free && ce[a] != cf[a];
+            }
+            if (free) break;
+        }
+        if (g == count.size()) {
+            count.push_back(0);
+            t.place.resize(count.size() * HT_GROUP, -1);
+        }
+        t.place[g * HT_GROUP + count[g]++] = e;
+    }
+}
+
+}  // namespace
+
+// The tiles of a model on the host; empty where fewer than min_nodes nodes have hex8 rows
+void hex_tiles_host(const Model &m, long long min_nodes, HexTilesHost &H) {
+    // node -> incident hex8 elements; nodes whose row is a sum of hex8 elements only
+    std::vector<int> off((size_t)m.nn + 1, 0);
+    std::vector<char> other((size_t)m.nn, 0);
+    for (int e : m.fe)
+        for (int a = 0; a < m.nen[e]; a++) {
+            const int k = m.econ[(size_t)e * 8 + a];
+            if (m.nen[e] == 8) off[k + 1]++;
+            else other[k] = 1;
+        }
+    std::vector<int> nodes;
+    for (int k = 0; k < m.nn; k++) {
+        if (off[k + 1] > 0 && !other[k] && m.famid[k] < 0) nodes.push_back(k);
+    }
+    if (nodes.empty() || (long long)nodes.size() < min_nodes) return;
+    std::partial_sum(off.begin(), off.end(), off.begin());
+    std::vector<int> inc((size_t)off[m.nn]);
+    {
+        std::vector<int> fill(off.begin(), off.end() - 1);
+        for (int e : m.fe)
+            if (m.nen[e] == 8)
+                for (int a = 0; a < 8; a++) inc[fill[m.econ[(size_t)e * 8 + a]]++] = e;
+    }
+    // mean node spacing, from the volume of the elements around the nodes
+    double vol = 0.0;
+    for (int k : nodes) vol += m.nv[k];
+    const double sp = std::cbrt(vol / (double)nodes.size()), width = 5.0 * sp;
+    std::vector<size_t> xs, ys;
+    cut_even(nodes, 0, nodes.size(), m.x.data(), 0, width, xs);
+    std::vector<std::vector<HostTile>> per_slab(xs.size() - 1);
+#pragma omp parallel private(ys)
+    {
+    // number of the last tile that took the element / node, and the element's or node's count in it
+    std::vector<int> in_e((size_t)m.ne, -1), in_n((size_t)m.nn, -1);
+    std::vector<unsigned short> loc((size_t)m.nn);  // local number of a node of the current tile
+    int serial = 0;
+#pragma omp for schedule(dynamic, 1)
+    for (int s = 0; s < (int)xs.size() - 1; s++) {
+        cut_even(nodes, xs[s], xs[s + 1], m.x.data(), 1, width, ys);
+        for (size_t q = 0; q + 1 < ys.size(); q++) {
+            sort_along(nodes, ys[q], ys[q + 1], m.x.data(), 2);
+            size_t at = ys[q];
+            while (at < ys[q + 1]) {
+                HostTile t;
+                serial++;
+                size_t end = at, layer = at, ne = 0, nn = 0;
+                for (size_t k = at; k < ys[q + 1]; k++) {
+                    const int nd = nodes[k];
+                    if (k > at && m.x[(size_t)nd * 3 + 2] - m.x[(size_t)nodes[k - 1] * 3 + 2] > 0.3 * sp) layer = k;
+                    size_t add = 0;
+                    for (int j = off[nd]; j < off[nd + 1]; j++) add += in_e[inc[j]] != serial;
+                    // eight new nodes per new element at most
+                    if (ne + add > (size_t)HT_ELE || k - at + 1 > (size_t)HT_OWN || nn + 8 * add > (size_t)HT_NODES) break;
+                    for (int j = off[nd]; j < off[nd + 1]; j++) {
+                        const int e = inc[j];
+                        if (in_e[e] == serial) continue;
+                        in_e[e] = serial;
+                        ne++;
+                        for (int a = 0; a < 8; a++) {
+                            int &v = in_n[m.econ[(size_t)e * 8 + a]];
+                            nn += v != serial;
+                            v = serial;
+                        }
+                    }
+                    end = k + 1;
+                }
+                if (end == at) break;  // a node of more elements than a tile holds: left to its row of K
+                // end on a layer of nodes where that keeps most of the tile
+                if (end < ys[q + 1] && layer > at && layer < end && layer - at >= (end - at) * 6 / 10) end = layer;
+                // the owned nodes, then the other nodes of their elements, each part in node order
+                t.node.assign(nodes.begin() + at, nodes.begin() + end);
+                std::sort(t.node.begin(), t.node.end());
+                t.n_own = int(t.node.size());
+                for (int nd : t.node) t.ele.insert(t.ele.end(), inc.begin() + off[nd], inc.begin() + off[nd + 1]);
+                std::sort(t.ele.begin(), t.ele.end());
+                t.ele.erase(std::unique(t.ele.begin(), t.ele.end()), t.ele.end());
+                serial++;
+                for (int nd : t.node) in_n[nd] = serial;
+                for (int e : t.ele)
+                    for (int a = 0; a < 8; a++) {
+                        const int v = m.econ[(size_t)e * 8 + a];
+                        if (in_n[v] == serial) continue;
+                        in_n[v] = serial;
+                        t.node.push_back(v);
+                    }
+                std::sort(t.node.begin() + t.n_own, t.node.end());
+                for (size_t i = 0; i < t.node.size(); i++) loc[t.node[i]] = (unsigned short)i;
+                place_elements(m, t);
+                t.conn.assign(t.place.size() * 8, 0xffff);
+                for (size_t i = 0; i < t.place.size(); i++)
+                    for (int a = 0; a < 8 && t.place[i] >= 0; a++) t.conn[i * 8 + a] = loc[m.econ[(size_t)t.place[i] * 8 + a]];
+                per_slab[s].push_back(std::move(t));
+                at = end;
+            }
+        }
+    }
+    }
+    std::vector<char> owned((size_t)m.nn, 0);
+    for (auto &slab : per_slab)
+        for (auto &t : slab) {
+            HexTile h{};
+            h.node0 = (int)H.nodes.size();
+            h.n_node = (int)t.node.size();
+            h.ele0 = (int)(H.conn.size() / 8);
+            h.n_ele = (int)t.place.size();
+            h.n_own = t.n_own;
+            for (int i = 0; i < t.n_own; i++) owned[t.node[i]] = 1;
+            for (int c = 0; c < 3; c++) h.x[c] = m.x[(size_t)t.node[0] * 3 + c];
+            H.nodes.insert(H.nodes.end(), t.node.begin(), t.node.end());
+            H.conn.insert(H.conn.end(), t.conn.begin(), t.conn.end());
+            H.tile.push_back(h);
+        }
+    // families of nodes without elements and without boundary terms, and the rows left to K
+    std::vector<char> edge((size_t)m.nn, 0);
+    for (int p = 0; p < m.npdbe; p++)
+        for (int a = 0; a < 4; a++) edge[m.pdbe[(size_t)p * 4 + a]] = 1;
+    for (int k = 0; k < m.nn; k++) {
+        if (owned[k]) continue;
+        if (m.famid[k] >= 0 && !edge[k] && !other[k] && off[k + 1] == off[k]) H.fams.push_back(m.famid[k]);
+        else H.rows.push_back(k);
+    }
+    // each XCD's list: its eighth of the tiles, families and rows, evenly mixed
+    const int n[3] = {(int)H.tile.size(), int(H.fams.size() + HEX_FAMS - 1) / HEX_FAMS,
+                      int(H.rows.size() + HEX_ROWS - 1) / HEX_ROWS};
+    std::vector<std::vector<HexTile>> list(8);
+    size_t per = 0;
+    for (int x = 0; x < 8; x++) {
+        std::vector<std::pair<double, HexTile>> l;
+        for (int kind = 0; kind < 3; kind++) {
+            const int b = int((long long)n[kind] * x / 8), e = int((long long)n[kind] * (x + 1) / 8);
+            for (int k = b; k < e; k++) {
+                HexTile w{};
+                if (kind == 0) {
+                    w = H.tile[k];
+                } else {
+                    const int size = kind == 1 ? HEX_FAMS : HEX_ROWS, all = int(kind == 1 ? H.fams.size() : H.rows.size());
+                    w.n_own = kind == 1 ? -1 : 0;
+                    w.node0 = k * size;
+                    w.n_node = std::min(size, all - w.node0);
+                }
+                l.push_back({(k - b + 0.5) / (e - b), w});
+            }
+        }
+        std::stable_sort(l.begin(), l.end(), [](const auto &a, const auto &b) { return a.first < b.first; });
+        for (auto &w : l) list[x].push_back(w.second);
+        per = std::max(per, l.size());
+    }
+    H.work.assign(per * 8, HexTile{});
+    for (int x = 0; x < 8; x++)
+        for (size_t q = 0; q < list[x].size(); q++) H.work[q * 8 + x] = list[x][q];
+}
+
+int hex_tiles(Ctx &c, const HexTiles *&out, std::string &err) {
+    out = (const HexTiles *)c.hex;
+    if (c.hex_tried) return PDX_OK;
+    HexTilesHost H;
+    if (c.dim == 3 && c.host && c.host->dim == 3) hex_tiles_host(*c.host, HEX_MIN_NODES, H);
+    if (H.tile.empty()) {
+        c.hex_tried = true;
+        return PDX_OK;
+    }
+    auto *T = new HexTiles();
+    c.hex = T;
+    T->n_work = (int)H.work.size();
+    T->n_fam = (int)H.fams.size();
+    auto up = [&](auto *&dst, const auto &src) -> int {
+        PDX_HIP(hipMalloc((void **)&dst, std::max<size_t>(src.size(), 1) * sizeof(src[0])));
+        if (!src.empty()) PDX_HIP(hipMemcpy(dst, src.data(), src.size() * sizeof(src[0]), hipMemcpyHostToDevice));
+        return PDX_OK;
+    };
+    int rc;
+    if ((rc = up(T->nodes, H.nodes)) || (rc = up(T->conn, H.conn)) ||
+        (rc = up(T->rows, H.rows)) ||
+        (rc = up(T->work, H.work)) || (rc = up(T->fams, H.fams))) {
+        free_hex_tiles(c);
+        return rc;
+    }
+    c.hex_tried = true;
+    out = T;
+    return PDX_OK;
+}
+
+void free_hex_tiles(Ctx &c) {
+    auto *T = (HexTiles *)c.hex;
+    if (!T) return;
+    for (void *p : {(void *)T->nodes, (void *)T->conn, (void *)T->rows, (void *)T->work, (void *)T->fams})
+        if (p) hipFree(p);
+    delete T;
+    c.hex = nullptr;
+    c.hex_tried = false;
+}
+
+}  // namespace pdx

@@ -16,6 +16,7 @@
 #include <functional>
 
 #include "device.hpp"
+#include "hex.hpp"
 #include "reduce.hpp"
 #include "rowblock.hpp"
 
@@ -120,6 +121,87 @@ __global__ void __launch_bounds__(256) k_explicit(const int *rows_s, int ns, int
         } else {
             Unp1[o] = un + inc;
         }
+    }
+}
+
+// The same step without most of K: the rows of the nodes whose elements are all hex8 are formed from
+// the elements, those of the interior PD nodes from the moments of their families (hex.hpp), FP64 in
+// both precisions; the other rows (PD boundary and tetrahedron nodes) are walked in K, a wavefront
+// each, in the same launch.  On the 60^3 box (198,520 elements, 8,000 PD nodes) the step takes 44 us
+// where the best walk of K takes 75 in FP64 (80^3: 86 against 195, 100^3: 173 against 389), and 45 in
+// FP32: K is 330 MB (196 MB) per step there, while the elements are 8.6M FP64 wavefront instructions (15 us at the full rate) on some 60 MB.  Bound by
+// those two one after the other: two workgroups of 198 registers fit a CU, and the ones in flight load
+// together and calculate together.
+template <typename T, bool FO>
+__global__ void __launch_bounds__(HT_THREADS, HT_WAVES) k_explicit_hex(
+    HexTiles ht, MomentArgs ma, double lam8, double mu8, const int *adj_off, const int *adj, const T *K,
+    const double *x, const double *Un, const double *Unm1, double *Unp1, const double *m, const double *f_unit, int n_nbc,
+    int nn, const double *nbc_cur, double *nbc_next, const double *nbc_inc, const int *eq, const int *presc_set,
+    const double *ebc_inc, double dt, int startup) {
+    __shared__ __align__(16) double lds[HT_LDS];
+    if (blockIdx.x == 0)
+        for (int s = threadIdx.x; s < n_nbc; s += blockDim.x) nbc_next[s] = nbc_cur[s] + nbc_inc[s];
+    // state of DOF i of node r, and its update when the row of K u_n is v
+    struct Dof {
+        size_t o;
+        int eq;
+        double unm1, m, fext;
+    };
+    auto load = [&](int r, int i) {
+        Dof d;
+        d.o = (size_t)r * 3 + i;
+        d.eq = eq[d.o];
+        d.m = FO ? 1.0 : m[d.o];
+        d.unm1 = FO ? 0.0 : Unm1[d.o];
+        d.fext = 0.0;
+        for (int s = 0; s < n_nbc; s++) d.fext = d.fext + nbc_cur[s] * f_unit[(size_t)s * nn * 3 + d.o];
+        return d;
+    };
+    auto update = [&](const Dof &d, double un, double v) {
+        const double F = d.fext - v;
+        double y;
+        if (d.eq < 0) y = FO ? 0.0 : un + ebc_inc[presc_set[d.o]];
+        else if (FO) y = F;
+        else if (startup) y = F / d.m * (0.5 * dt * dt) + un;
+        else y = un * 2.0 + dt * dt * F / d.m - d.unm1;
+        Unp1[d.o] = y;
+    };
+    const HexTile t = ht.work[blockIdx.x];
+    if (t.n_own > 0) {
+        hex_tile_product<double, double, false>(t, ht, x, Un, lam8, mu8, 0.0, lds);
+        // the owned DOFs' state is on its way while the last wavefronts still add
+        constexpr int ND = (HT_OWN * 3 + HT_THREADS - 1) / HT_THREADS;
+        Dof d[ND];
+#pragma unroll
+        for (int q = 0; q < ND; q++) {
+            const int k = threadIdx.x + q * HT_THREADS, n = k / 3;
+            if (n < t.n_own) d[q] = load(ht.nodes[t.node0 + n], k - n * 3);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < ND; q++) {
+            const int k = threadIdx.x + q * HT_THREADS, n = k / 3;
+            if (n < t.n_own) update(d[q], hex_tile_u(lds, n, k - n * 3), hex_tile_sum(lds, k));
+        }
+    } else if (t.n_own < 0) {
+        const int q = threadIdx.x / 16, lane = threadIdx.x % 16;
+        if (q >= t.n_node) return;
+        const int f = ht.fams[t.node0 + q];
+        double v[3];
+        family_row(ma, f, lane, x, Un, v);
+        if (lane < 3) {
+            const Dof d = load(ma.fam_mem[ma.fam_off[f]], lane);
+            update(d, Un[d.o], pick<3, double>(v, lane));
+        }
+    } else {
+        const int q = threadIdx.x / 64, lane = threadIdx.x % 64;
+        if (q >= t.n_node) return;
+        const int row = ht.rows[t.node0 + q];
+        Dof d;
+        if (lane < 3) d = load(row, lane);
+        T acc[3];
+        row_matvec<3, T, double, 64, sizeof(T) == 4>(row, lane, adj_off, adj, K, Un, acc);
+        if (lane < 3) update(d, Un[d.o], double(pick<3, T>(acc, lane)));
     }
 }
 
@@ -373,6 +455,27 @@ static void launch_explicit_any(Ctx &c, int prec, int variant, const double *Un,
     }
 }
 
+// FP32 steps walk K up to this many nodes: its 4-byte values stay in the 256 MB Infinity Cache so
+// long (31^3 nodes: 9.5 us against 11.7 through the tiles; 60^3: 44.8 against 44.0, for a longer
+// first call; 66^3: 58.3 against 55.8; 80^3: 124 against 86)
+constexpr int HEX_MIN_NODES_F32 = 262144;
+
+// the tiles a step of precision index pi goes through, or null when it walks K in one of the forms
+// (a form set by the caller, or no tiles for this model)
+static int step_tiles(Ctx &c, int pi, const HexTiles *&ht, std::string &err) {
+    ht = nullptr;
+    if (c.tune_explicit[pi] >= 0 || (pi && c.nn < HEX_MIN_NODES_F32)) return PDX_OK;
+    return hex_tiles(c, ht, err);
+}
+
+template <typename T, bool FO>
+static void launch_explicit_hex(Ctx &c, const HexTiles &ht, const T *K, const double *Un, const double *Unm1,
+                                double *Unp1, const double *nbc_cur, double *nbc_next, int startup) {
+    k_explicit_hex<T, FO><<<ht.n_work, HT_THREADS, 0, c.stream>>>(
+        ht, moment_args(c), c.lambda / 8, c.mu / 8, c.adj_off, c.adj, K, c.x, Un, Unm1, Unp1, c.mlump, c.f_unit, c.n_nbc, c.nn,
+        nbc_cur, nbc_next, c.d_nbc_vel, c.eq, c.presc_set, c.d_ebc_vel, c.dt, startup);
+}
+
 // Autotuner: time every variant on the current state with the result written to
 // scratch buffers (the simulation state is not advanced), keep the fastest.
 static int tune_explicit(Ctx &c, int prec, std::string &err) {
@@ -415,8 +518,16 @@ static void explicit_step(Ctx &c, int prec, int startup) {
     const long long s = startup ? 0 : c.steps_done + 1;
     double *nbc_cur = c.nbcv + (s % 2) * std::max(c.n_nbc, 1);
     double *nbc_next = c.nbcv + ((s + 1) % 2) * std::max(c.n_nbc, 1);
-    launch_explicit_any(c, prec, std::max(c.tune_explicit[prec == PDX_FP32 ? 1 : 0], 0), Un, Unm1, Unp1, nbc_cur,
-                        nbc_next, startup, s);
+    const HexTiles *ht = nullptr;
+    std::string unused;  // the tiles, if any, were built by explicit_operators
+    step_tiles(c, prec == PDX_FP32 ? 1 : 0, ht, unused);
+    if (ht && prec == PDX_FP32)
+        launch_explicit_hex<float, false>(c, *ht, c.K32, Un, Unm1, Unp1, nbc_cur, nbc_next, startup);
+    else if (ht)
+        launch_explicit_hex<double, false>(c, *ht, c.K, Un, Unm1, Unp1, nbc_cur, nbc_next, startup);
+    else
+        launch_explicit_any(c, prec, std::max(c.tune_explicit[prec == PDX_FP32 ? 1 : 0], 0), Un, Unm1, Unp1, nbc_cur,
+                            nbc_next, startup, s);
     c.step_phase = (p + 1) % 3;
     c.steps_done = s;
 }
@@ -490,8 +601,15 @@ static int explicit_operators(Ctx &c, int prec, bool lumped, std::string &err) {
         int e = ensure_K32(c, err);
         if (e) return e;
     }
-    if (int e = ensure_Ks(c, prec, err)) return e;
-    if (int e = ensure_Kown(c, prec, err)) return e;
+    const HexTiles *ht = nullptr;
+    if (int e = step_tiles(c, prec == PDX_FP32 ? 1 : 0, ht, err)) return e;
+    if (ht) {
+        if (ht->n_fam)
+            if (int e = dev_family_moments(c, err)) return e;
+    } else {
+        if (int e = ensure_Ks(c, prec, err)) return e;
+        if (int e = ensure_Kown(c, prec, err)) return e;
+    }
     if (lumped && !c.mlump_valid) {
         int e = dev_lumped_mass(c, err);
         if (e) return e;
@@ -566,11 +684,26 @@ int dev_explicit_dofvals(Ctx &c, const double **out, std::string &err) {
 
 int explicit_tune_if_needed(Ctx &c, int prec, std::string &err) {
     const int pi = prec == PDX_FP32 ? 1 : 0;
-    if (c.tune_explicit[pi] >= 0) return PDX_OK;
-    int rc = tune_explicit(c, pi, err);
+    const HexTiles *ht = nullptr;
+    int rc = step_tiles(c, pi, ht, err);
+    if (rc || ht || c.tune_explicit[pi] >= 0) return rc;
+    rc = tune_explicit(c, pi, err);
     for (auto &g : c.graph)
         if (g) { hipGraphExecDestroy(g); g = nullptr; }
     return rc;
+}
+
+// What pdx_explicit_tuning reports for a context that steps through the tiles: the fastest K form
+// for its current state, timed when first asked for (the steps stay on the tiles)
+int explicit_tune_seen(Ctx &c, int pi, std::string &err) {
+    if (c.tune_explicit[pi] >= 0 || c.tune_seen[pi] >= 0 || !c.hex || c.steps_done < 0) return PDX_OK;
+    const int prec = pi ? PDX_FP32 : PDX_FP64;
+    if (!c.K_valid || (pi && !c.K32_valid)) return PDX_OK;
+    int rc;
+    if ((rc = ensure_Ks(c, prec, err)) || (rc = ensure_Kown(c, prec, err)) || (rc = tune_explicit(c, pi, err))) return rc;
+    c.tune_seen[pi] = c.tune_explicit[pi];
+    c.tune_explicit[pi] = -1;
+    return PDX_OK;
 }
 
 // Capture the 6-step graph of precision prec (three rotating state vectors, two NBC buffers:

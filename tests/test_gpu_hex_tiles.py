@@ -1,0 +1,98 @@
+"""The products with hex8 elements and PD families without their blocks of K (csrc/hex.hip) against the walk of K.
+
+Both sum the same terms in FP64 in another order, so a trajectory differs by rounding only: a product of a row of some
+30 to 130 blocks of 3 x 3 carries at most about 400 roundings of 1.1e-16 of its absolute terms, 5e-14, and the
+differences of 25 steps stay below 25 times that: 1e-12.  The meshes lie above the size from which the tiles are used.
+"""
+import numpy as np
+import pytest
+
+from helpers import load_pdx, rel, workloads
+
+pytestmark = pytest.mark.gpu
+pdx, W = load_pdx(), workloads()
+
+
+def _dt(mesh):
+    mesh["dt"] = 2e-8  # 1 mm elements of steel-like stiffness: a fraction of the critical step
+    mesh["nbc"][0].update(vel=1e12, vary=True)
+    mesh["ebc"][0].update(vel=1e-3, vary=True)
+    return mesh
+
+
+def _shuffled(mesh, seed=0):
+    """The same body with its nodes renumbered and every element started at another corner."""
+    rng = np.random.default_rng(seed)
+    p = rng.permutation(len(mesh["x"]))
+    inv = np.argsort(p)
+    e = inv[np.asarray(mesh["econ"]) - 1] + 1
+    turn, tip = [1, 2, 3, 0, 5, 6, 7, 4], [3, 2, 6, 7, 0, 1, 5, 4]
+    for k in range(len(e)):
+        if mesh["algo"][k] == 2:  # the PD elements' faces are matched by their corner order
+            for _ in range(rng.integers(4)):
+                e[k] = e[k][turn]
+            for _ in range(rng.integers(4)):
+                e[k] = e[k][tip]
+    mesh["x"], mesh["econ"] = np.asarray(mesh["x"])[p], e.astype(np.int32)
+    for s in mesh["ebc"]:
+        s["nid"] = inv[np.asarray(s["nid"]) - 1] + 1
+    for s in mesh["nbc"]:
+        s["con"] = inv[np.asarray(s["con"]) - 1] + 1
+    return mesh
+
+
+def _with_tets(mesh, share=0.02):
+    """Some of the FE hexahedra split into five tetrahedra each."""
+    rng = np.random.default_rng(1)
+    econ, nen, algo = np.asarray(mesh["econ"]), np.asarray(mesh["nen"]), np.asarray(mesh["algo"])
+    split = (algo == 2) & (rng.random(len(econ)) < share)
+    five = [(0, 1, 2, 5), (0, 2, 3, 7), (0, 5, 7, 4), (2, 7, 5, 6), (0, 2, 7, 5)]
+    t = np.zeros((5 * int(split.sum()), 8), np.int32)
+    t[:, :4] = np.concatenate([econ[split][:, list(q)] for q in five])
+    mesh["econ"] = np.concatenate([econ[~split], t])
+    mesh["nen"] = np.concatenate([nen[~split], np.full(len(t), 4, np.int32)])
+    mesh["algo"] = np.concatenate([algo[~split], np.full(len(t), 2, np.int32)])
+    return mesh
+
+
+CASES = {
+    "pd_block": lambda: W.box3d(n=31, pd_block=9),
+    "elements_only": lambda: W.box3d(n=29, pd_block=0),
+    "shuffled": lambda: _shuffled(W.box3d(n=30, pd_block=8)),
+    "with_tets": lambda: _with_tets(W.box3d(n=33, pd_block=8)),
+    "penny_crack": lambda: W.penny3d(n=32, pd_block=8),
+}
+
+
+@pytest.mark.parametrize("name", list(CASES))
+def test_explicit_through_tiles_equals_walk_of_K(name):
+    model = pdx.Model(_dt(CASES[name]()))
+    tiles, walk = pdx.Context(model), pdx.Context(model)
+    walk.explicit_set_form(pdx.PDX_FP64, 0)
+    for steps in (1, 24):
+        (u, up), (v, vp) = tiles.explicit_run(steps), walk.explicit_run(steps)
+        assert np.linalg.norm(v) > 0
+        assert rel(u, v) <= 1e-12 and rel(up, vp) <= 1e-12
+    # the sums have one order: eager steps of another context give the same bits as the replayed ones
+    eager = pdx.Context(model)
+    eager.explicit_steps(25, use_graph=False)
+    assert np.array_equal(eager.explicit_run(0)[0], u)
+    # a form can still be set, and taken back, between steps; the tuning is reported as before
+    tiles.explicit_set_form(pdx.PDX_FP64, 21)
+    assert rel(tiles.explicit_run(6)[0], walk.explicit_run(6)[0]) <= 1e-12
+    tiles.explicit_set_form(pdx.PDX_FP64, -1)
+    assert rel(tiles.explicit_run(6)[0], walk.explicit_run(6)[0]) <= 1e-12
+    assert 0 <= tiles.explicit_tuning_full(pdx.PDX_FP64)[8] < pdx.EXPLICIT_FORMS
+    assert rel(tiles.explicit_run(6)[0], walk.explicit_run(6)[0]) <= 1e-12
+
+
+def test_fp32_force_through_tiles():
+    """FP32 force (large models only): the tiles calculate in FP64, so they are no further from FP64 than the walk."""
+    model = pdx.Model(_dt(W.box3d(n=65, pd_block=12)))
+    ref, tiles, walk = (pdx.Context(model) for _ in range(3))
+    ref.explicit_set_form(pdx.PDX_FP64, 0)
+    walk.explicit_set_form(pdx.PDX_FP32, 0)
+    u = ref.explicit_run(25)[0]
+    e_tiles = rel(tiles.explicit_run(25, pdx.PDX_FP32)[0], u)
+    e_walk = rel(walk.explicit_run(25, pdx.PDX_FP32)[0], u)
+    assert e_tiles <= 1.2 * e_walk <= 1e-6
