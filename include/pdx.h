@@ -148,7 +148,8 @@ typedef struct pdx_solve_opts {
                           each lower block that no family stores in either orientation read as its
                           upper partner's transpose, once a device check has found every such block
                           equal to that transpose bit for bit (else full storage; same results, bit
-                          for bit, either way) */
+                          for bit, either way).  Products of large 3D models that are formed from the
+                          elements and families instead of from the operator's blocks read neither */
 } pdx_solve_opts;
 
 typedef struct pdx_solve_stats {
@@ -160,7 +161,8 @@ typedef struct pdx_solve_stats {
     int precond_used;   /* PDX_PREC_* of the attempt that ended the solve */
     int precision_used; /* PDX_FP64 / PDX_FP32 of that attempt */
     int attempts;       /* 1 + fallback retries */
-    int mirrored_used;  /* 1 when the SpMVs read mirrored storage (pdx_solve_opts.mirrored) */
+    int mirrored_used;  /* 1 when the SpMVs read mirrored storage (pdx_solve_opts.mirrored); 0 too where
+                           they do not read the operator's blocks */
 } pdx_solve_stats;
 
 const char *pdx_last_error(void);
@@ -409,13 +411,16 @@ int pdx_last_timing(pdx_ctx *c, double *total_ms, double *per_step_ms);
  * from element matrices only) is read from the partner's storage; alternating: every other step
  * visits the rows last to first, so a step begins on the data the previous one read last (forms
  * 20-23); all 0 before the first step)
- * and its timings of the PDX_EXPLICIT_FORMS forms (ms per step) */
+ * and its timings of the PDX_EXPLICIT_FORMS forms (ms per step).  A context of a large 3D model steps
+ * without walking most of K (rows of hex8 nodes from the elements, of interior PD nodes from their
+ * families) while no form is set: the forms are then timed when this is called, and the fastest is
+ * reported, not used */
 #define PDX_EXPLICIT_FORMS 24
 int pdx_explicit_tuning(pdx_ctx *c, int precision, int *lanes, int *nontemporal, int *xcd_order, int *row_soa,
                         int *col_classes, int *mirrored, int *alternating, int *form,
                         float *ms /*[PDX_EXPLICIT_FORMS]*/);
 /* use explicit-step form `form` (0 .. PDX_EXPLICIT_FORMS-1) from now on instead of the tuner's
- * choice, or -1 to tune again at the next step; forms with the same lanes per row compute the
+ * choice (or the products without K), or -1 to choose again at the next step; forms with the same lanes per row compute the
  * same bits, the lanes per row change the order of the row sum */
 int pdx_explicit_set_form(pdx_ctx *c, int precision, int form);
 

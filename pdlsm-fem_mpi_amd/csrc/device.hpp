@@ -169,6 +169,7 @@ struct Ctx {
     // node tiles of the products with hex8 elements without their K blocks (hex.hip)
     void *hex = nullptr;
     bool hex_tried = false;
+    std::vector<int> nfe_off_host, nfe_item_host;  // nfe_off, nfe_item (3D), until the tiles are built
     // PD rows formed from the moments of their families (hex.hpp): bond weights [members] and the
     // second-order rows of the inverse shape tensors [nfam * 54], for the K of generation mom_gen
     double *mom_w = nullptr, *mom_T = nullptr;
@@ -177,7 +178,8 @@ struct Ctx {
 
     // scratch for Krylov
     std::vector<DevBuf> scratch;
-    double *red = nullptr;      // partial sums [RED_SLOTS * RED_PARTS]
+    double *red = nullptr;      // partial sums [RED_SLOTS * RED_PARTS], scalars, per-block partials [2 * red_blocks]
+    int red_blocks = 0;
     double *red_host = nullptr; // pinned mirror
     double last_total_ms = 0, last_step_ms = 0;
     void *two_level = nullptr;       // coarse space of the last two-level solve (krylov.hip)
@@ -234,6 +236,9 @@ int dev_spmv_K(Ctx &c, const double *K64, const double *x, double *y);
 struct Mirrored {
     const double *K64 = nullptr;
     const float *K32 = nullptr;
+    // the operator is ks K + ms M (M: the consistent mass) of this context, so that its products may be
+    // formed from the elements and families (hex.hpp); ks = 0: some other matrix
+    double ks = 0.0, ms = 0.0;
 };
 // exact: every mirrored lower block of A (dd*nblk values, K's block order) equals its partner's
 // transpose bit for bit (checked on the device; synchronises the stream)
@@ -242,6 +247,10 @@ int check_mirrored(Ctx &c, const double *A, bool &exact, std::string &err);
 int gather_own(Ctx &c, const double *A, double *own64, float *own32, std::string &err);
 // mirrored copies of the context's K for a solve in precision prec (empty when not exact)
 int kown_for_solve(Ctx &c, int prec, Mirrored &m, std::string &err);
+// whether a solve in precision prec with this context's operators goes through the tiles (hex.hpp), and the
+// FP64 product with K through them
+int dev_product_tiles(Ctx &c, int prec, bool &tiles, std::string &err);
+int dev_spmv_tiles(Ctx &c, const double *x, double *y, std::string &err);
 int dev_solve_mat(Ctx &c, const double *K64, const float *K32, const pdx_solve_opts &o, const double *b_dev,
                   double *x_dev, pdx_solve_stats &st, std::string &err, const Mirrored *mir = nullptr);
 void free_two_level(Ctx &c);

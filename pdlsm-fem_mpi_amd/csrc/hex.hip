@@ -2,6 +2,8 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
+#include <bitset>
 #include <cmath>
 #include <cstring>
 #include <numeric>
@@ -20,6 +22,7 @@ struct HostTile {
     std::vector<unsigned short> conn;
 };
 
+// v[b, e) by coordinate, then node
 void sort_along(std::vector<int> &v, size_t b, size_t e, const double *x, int axis) {
     std::vector<std::pair<double, int>> k(e - b);
     for (size_t i = b; i < e; i++) k[i - b] = {x[(size_t)v[i] * 3 + axis], v[i]};
@@ -27,12 +30,39 @@ void sort_along(std::vector<int> &v, size_t b, size_t e, const double *x, int ax
     for (size_t i = b; i < e; i++) v[i] = k[i - b].second;
 }
 
+// the same for a long list: equal bins of the coordinate range, each sorted by itself
+void sort_along_parallel(std::vector<int> &v, const double *x, int axis) {
+    constexpr int NB = 1024;
+    const size_t n = v.size();
+    double lo = 1e300, hi = -1e300;
+#pragma omp parallel for schedule(static) reduction(min : lo) reduction(max : hi)
+    for (size_t i = 0; i < n; i++) {
+        const double c = x[(size_t)v[i] * 3 + axis];
+        lo = std::min(lo, c);
+        hi = std::max(hi, c);
+    }
+    const double scale = hi > lo ? NB / (hi - lo) : 0.0;
+    auto bin = [&](int k) { return std::min(NB - 1, std::max(0, int((x[(size_t)k * 3 + axis] - lo) * scale))); };
+    std::vector<unsigned short> at(n);
+#pragma omp parallel for schedule(static)
+    for (size_t i = 0; i < n; i++) at[i] = (unsigned short)bin(v[i]);
+    std::vector<size_t> off(NB + 1, 0);
+    for (size_t i = 0; i < n; i++) off[at[i] + 1]++;
+    for (int i = 0; i < NB; i++) off[i + 1] += off[i];
+    std::vector<size_t> fill(off.begin(), off.end() - 1);
+    std::vector<int> out(n);
+    for (size_t i = 0; i < n; i++) out[fill[at[i]]++] = v[i];
+    v.swap(out);
+#pragma omp parallel for schedule(dynamic, 8)
+    for (int i = 0; i < NB; i++) sort_along(v, off[i], off[i + 1], x, axis);
+}
+
 // Nodes in slabs along x, the slabs in columns along y, each about `w` node spacings wide, the cuts
-// moved to the widest gap between neighbouring coordinates near the even position (so that a mesh
+// (v[b, e) is sorted along the axis) moved to the widest gap between neighbouring coordinates near the even position (so that a mesh
 // with layers is cut between layers); a column is then filled from below, node by node in z, until a
 // tile is full.
-void cut_even(std::vector<int> &v, size_t b, size_t e, const double *x, int axis, double width, std::vector<size_t> &cuts) {
-    sort_along(v, b, e, x, axis);
+void cut_even(const std::vector<int> &v, size_t b, size_t e, const double *x, int axis, double width,
+              std::vector<size_t> &cuts) {
     cuts.assign(1, b);
     const size_t n = e - b;
     const double ext = n ? x[(size_t)v[e - 1] * 3 + axis] - x[(size_t)v[b] * 3 + axis] : 0.0;
@@ -54,88 +84,95 @@ void cut_even(std::vector<int> &v, size_t b, size_t e, const double *x, int axis
 }
 
 // Elements into groups of HT_GROUP, in order, none beside another with the same node in the same
-// corner (two elements of a consistently numbered mesh never are)
-void place_elements(const Model &m, HostTile &t) {
-    std::vector<int> count;  // elements of each group
+// corner (two elements of a consistently numbered mesh never are); loc: local number of a node
+void place_elements(const Model &m, const std::vector<unsigned short> &loc, HostTile &t) {
+    using Used = std::bitset<HT_NODES>;
+    std::vector<std::array<Used, 8>> used;  // nodes in each corner of each group
+    std::vector<int> count;                 // elements of each group
+    size_t first = 0;                       // the first group with a place left
     t.place.clear();
     for (int e : t.ele) {
-        const int *ce = &m.econ[(size_t)e * 8];
-        size_t g = 0;
+        unsigned short l[8];
+        for (int a = 0; a < 8; a++) l[a] = loc[m.econ[(size_t)e * 8 + a]];
+        while (first < count.size() && count[first] == HT_GROUP) first++;
+        size_t g = first;
         for (; g < count.size(); g++) {
-            if (count[g] == HT_GROUP) continue;
-            bool free = true;
-            for (int k = 0; k < count[g] && free; k++) {
-                const int *cf = &m.econ[(size_t)t.place[g * HT_GROUP + k] * 8];
-                for (int a = 0; a < 8; a++) free = free && ce[a] != cf[a];
-            }
+            bool free = count[g] < HT_GROUP;
+            for (int a = 0; a < 8 && free; a++) free = !used[g][a][l[a]];
             if (free) break;
         }
         if (g == count.size()) {
             count.push_back(0);
+            used.emplace_back();
             t.place.resize(count.size() * HT_GROUP, -1);
         }
+        for (int a = 0; a < 8; a++) used[g][a][l[a]] = true;
         t.place[g * HT_GROUP + count[g]++] = e;
     }
 }
 
 }  // namespace
 
-// The tiles of a model on the host; empty where fewer than min_nodes nodes have hex8 rows
-void hex_tiles_host(const Model &m, long long min_nodes, HexTilesHost &H) {
-    // node -> incident hex8 elements; nodes whose row is a sum of hex8 elements only
-    std::vector<int> off((size_t)m.nn + 1, 0);
-    std::vector<char> other((size_t)m.nn, 0);
-    for (int e : m.fe)
-        for (int a = 0; a < m.nen[e]; a++) {
-            const int k = m.econ[(size_t)e * 8 + a];
-            if (m.nen[e] == 8) off[k + 1]++;
-            else other[k] = 1;
-        }
-    std::vector<int> nodes;
+// The tiles of a model on the host (nfe_off, nfe_item: per node its FE elements in element order, as
+// FE position * 8 + corner); empty where fewer than min_nodes nodes have hex8 rows
+void hex_tiles_host(const Model &m, const std::vector<int> &nfe_off, const std::vector<int> &nfe_item, long long min_nodes,
+                    HexTilesHost &H) {
+    // nodes whose row is a sum of hex8 elements only
+    const std::vector<int> &off = nfe_off;
+    auto inc = [&](int j) { return m.fe[nfe_item[j] >> 3]; };
+    std::vector<char> hex((size_t)m.nn, 0);
+#pragma omp parallel for schedule(static)
     for (int k = 0; k < m.nn; k++) {
-        if (off[k + 1] > 0 && !other[k] && m.famid[k] < 0) nodes.push_back(k);
+        bool all = off[k + 1] > off[k] && m.famid[k] < 0;
+        for (int j = off[k]; j < off[k + 1] && all; j++) all = m.nen[inc(j)] == 8;
+        hex[k] = all;
     }
+    std::vector<int> nodes;
+    for (int k = 0; k < m.nn; k++)
+        if (hex[k]) nodes.push_back(k);
     if (nodes.empty() || (long long)nodes.size() < min_nodes) return;
-    std::partial_sum(off.begin(), off.end(), off.begin());
-    std::vector<int> inc((size_t)off[m.nn]);
-    {
-        std::vector<int> fill(off.begin(), off.end() - 1);
-        for (int e : m.fe)
-            if (m.nen[e] == 8)
-                for (int a = 0; a < 8; a++) inc[fill[m.econ[(size_t)e * 8 + a]]++] = e;
-    }
     // mean node spacing, from the volume of the elements around the nodes
     double vol = 0.0;
     for (int k : nodes) vol += m.nv[k];
     const double sp = std::cbrt(vol / (double)nodes.size()), width = 5.0 * sp;
-    std::vector<size_t> xs, ys;
+    std::vector<size_t> xs;
+    sort_along_parallel(nodes, m.x.data(), 0);
     cut_even(nodes, 0, nodes.size(), m.x.data(), 0, width, xs);
-    std::vector<std::vector<HostTile>> per_slab(xs.size() - 1);
-#pragma omp parallel private(ys)
-    {
-    // number of the last tile that took the element / node, and the element's or node's count in it
-    std::vector<int> in_e((size_t)m.ne, -1), in_n((size_t)m.nn, -1);
-    std::vector<unsigned short> loc((size_t)m.nn);  // local number of a node of the current tile
-    int serial = 0;
-#pragma omp for schedule(dynamic, 1)
+    // columns: the slabs cut along y, each sorted along z
+    std::vector<std::vector<size_t>> ys(xs.size() - 1);
+#pragma omp parallel for schedule(dynamic, 1)
     for (int s = 0; s < (int)xs.size() - 1; s++) {
-        cut_even(nodes, xs[s], xs[s + 1], m.x.data(), 1, width, ys);
-        for (size_t q = 0; q + 1 < ys.size(); q++) {
-            sort_along(nodes, ys[q], ys[q + 1], m.x.data(), 2);
-            size_t at = ys[q];
-            while (at < ys[q + 1]) {
+        sort_along(nodes, xs[s], xs[s + 1], m.x.data(), 1);
+        cut_even(nodes, xs[s], xs[s + 1], m.x.data(), 1, width, ys[s]);
+    }
+    std::vector<std::pair<size_t, size_t>> column;
+    for (auto &y : ys)
+        for (size_t q = 0; q + 1 < y.size(); q++) column.push_back({y[q], y[q + 1]});
+    std::vector<std::vector<HostTile>> per_column(column.size());
+#pragma omp parallel
+    {
+        // number of the last tile that took the element / node
+        std::vector<int> in_e((size_t)m.ne, -1), in_n((size_t)m.nn, -1);
+        std::vector<unsigned short> loc((size_t)m.nn);  // local number of a node of the current tile
+        int serial = 0;
+#pragma omp for schedule(dynamic, 1)
+        for (int q = 0; q < (int)column.size(); q++) {
+            const size_t last = column[q].second;
+            sort_along(nodes, column[q].first, last, m.x.data(), 2);
+            size_t at = column[q].first;
+            while (at < last) {
                 HostTile t;
                 serial++;
                 size_t end = at, layer = at, ne = 0, nn = 0;
-                for (size_t k = at; k < ys[q + 1]; k++) {
+                for (size_t k = at; k < last; k++) {
                     const int nd = nodes[k];
                     if (k > at && m.x[(size_t)nd * 3 + 2] - m.x[(size_t)nodes[k - 1] * 3 + 2] > 0.3 * sp) layer = k;
                     size_t add = 0;
-                    for (int j = off[nd]; j < off[nd + 1]; j++) add += in_e[inc[j]] != serial;
+                    for (int j = off[nd]; j < off[nd + 1]; j++) add += in_e[inc(j)] != serial;
                     // eight new nodes per new element at most
                     if (ne + add > (size_t)HT_ELE || k - at + 1 > (size_t)HT_OWN || nn + 8 * add > (size_t)HT_NODES) break;
                     for (int j = off[nd]; j < off[nd + 1]; j++) {
-                        const int e = inc[j];
+                        const int e = inc(j);
                         if (in_e[e] == serial) continue;
                         in_e[e] = serial;
                         ne++;
@@ -149,16 +186,22 @@ void hex_tiles_host(const Model &m, long long min_nodes, HexTilesHost &H) {
                 }
                 if (end == at) break;  // a node of more elements than a tile holds: left to its row of K
                 // end on a layer of nodes where that keeps most of the tile
-                if (end < ys[q + 1] && layer > at && layer < end && layer - at >= (end - at) * 6 / 10) end = layer;
-                // the owned nodes, then the other nodes of their elements, each part in node order
+                if (end < last && layer > at && layer < end && layer - at >= (end - at) * 6 / 10) end = layer;
+                // the owned nodes in node order, then the other nodes of their elements as these list them
                 t.node.assign(nodes.begin() + at, nodes.begin() + end);
                 std::sort(t.node.begin(), t.node.end());
                 t.n_own = int(t.node.size());
-                for (int nd : t.node) t.ele.insert(t.ele.end(), inc.begin() + off[nd], inc.begin() + off[nd + 1]);
-                std::sort(t.ele.begin(), t.ele.end());
-                t.ele.erase(std::unique(t.ele.begin(), t.ele.end()), t.ele.end());
                 serial++;
-                for (int nd : t.node) in_n[nd] = serial;
+                for (int nd : t.node) {
+                    in_n[nd] = serial;
+                    for (int j = off[nd]; j < off[nd + 1]; j++) {
+                        const int e = inc(j);
+                        if (in_e[e] == serial) continue;
+                        in_e[e] = serial;
+                        t.ele.push_back(e);
+                    }
+                }
+                std::sort(t.ele.begin(), t.ele.end());
                 for (int e : t.ele)
                     for (int a = 0; a < 8; a++) {
                         const int v = m.econ[(size_t)e * 8 + a];
@@ -166,40 +209,50 @@ void hex_tiles_host(const Model &m, long long min_nodes, HexTilesHost &H) {
                         in_n[v] = serial;
                         t.node.push_back(v);
                     }
-                std::sort(t.node.begin() + t.n_own, t.node.end());
                 for (size_t i = 0; i < t.node.size(); i++) loc[t.node[i]] = (unsigned short)i;
-                place_elements(m, t);
+                place_elements(m, loc, t);
                 t.conn.assign(t.place.size() * 8, 0xffff);
                 for (size_t i = 0; i < t.place.size(); i++)
                     for (int a = 0; a < 8 && t.place[i] >= 0; a++) t.conn[i * 8 + a] = loc[m.econ[(size_t)t.place[i] * 8 + a]];
-                per_slab[s].push_back(std::move(t));
+                per_column[q].push_back(std::move(t));
                 at = end;
             }
         }
     }
+    // flat arrays
+    std::vector<const HostTile *> all;
+    for (auto &col : per_column)
+        for (auto &t : col) all.push_back(&t);
+    H.tile.resize(all.size());
+    size_t n_node = 0, n_ele = 0;
+    for (size_t k = 0; k < all.size(); k++) {
+        HexTile h{};
+        h.node0 = (int)n_node;
+        h.n_node = (int)all[k]->node.size();
+        h.ele0 = (int)n_ele;
+        h.n_ele = (int)all[k]->place.size();
+        h.n_own = all[k]->n_own;
+        for (int c = 0; c < 3; c++) h.x[c] = m.x[(size_t)all[k]->node[0] * 3 + c];
+        n_node += all[k]->node.size();
+        n_ele += all[k]->place.size();
+        H.tile[k] = h;
     }
+    H.nodes.resize(n_node);
+    H.conn.resize(n_ele * 8);
     std::vector<char> owned((size_t)m.nn, 0);
-    for (auto &slab : per_slab)
-        for (auto &t : slab) {
-            HexTile h{};
-            h.node0 = (int)H.nodes.size();
-            h.n_node = (int)t.node.size();
-            h.ele0 = (int)(H.conn.size() / 8);
-            h.n_ele = (int)t.place.size();
-            h.n_own = t.n_own;
-            for (int i = 0; i < t.n_own; i++) owned[t.node[i]] = 1;
-            for (int c = 0; c < 3; c++) h.x[c] = m.x[(size_t)t.node[0] * 3 + c];
-            H.nodes.insert(H.nodes.end(), t.node.begin(), t.node.end());
-            H.conn.insert(H.conn.end(), t.conn.begin(), t.conn.end());
-            H.tile.push_back(h);
-        }
+#pragma omp parallel for schedule(static)
+    for (int k = 0; k < (int)all.size(); k++) {
+        std::copy(all[k]->node.begin(), all[k]->node.end(), H.nodes.begin() + H.tile[k].node0);
+        std::copy(all[k]->conn.begin(), all[k]->conn.end(), H.conn.begin() + (size_t)H.tile[k].ele0 * 8);
+        for (int i = 0; i < all[k]->n_own; i++) owned[all[k]->node[i]] = 1;
+    }
     // families of nodes without elements and without boundary terms, and the rows left to K
     std::vector<char> edge((size_t)m.nn, 0);
     for (int p = 0; p < m.npdbe; p++)
         for (int a = 0; a < 4; a++) edge[m.pdbe[(size_t)p * 4 + a]] = 1;
     for (int k = 0; k < m.nn; k++) {
         if (owned[k]) continue;
-        if (m.famid[k] >= 0 && !edge[k] && !other[k] && off[k + 1] == off[k]) H.fams.push_back(m.famid[k]);
+        if (m.famid[k] >= 0 && !edge[k] && off[k + 1] == off[k]) H.fams.push_back(m.famid[k]);
         else H.rows.push_back(k);
     }
     // each XCD's list: its eighth of the tiles, families and rows, evenly mixed
@@ -237,7 +290,9 @@ int hex_tiles(Ctx &c, const HexTiles *&out, std::string &err) {
     out = (const HexTiles *)c.hex;
     if (c.hex_tried) return PDX_OK;
     HexTilesHost H;
-    if (c.dim == 3 && c.host && c.host->dim == 3) hex_tiles_host(*c.host, HEX_MIN_NODES, H);
+    if (c.dim == 3 && c.host && c.host->dim == 3) hex_tiles_host(*c.host, c.nfe_off_host, c.nfe_item_host, HEX_MIN_NODES, H);
+    c.nfe_off_host = std::vector<int>();
+    c.nfe_item_host = std::vector<int>();
     if (H.tile.empty()) {
         c.hex_tried = true;
         return PDX_OK;

@@ -14,7 +14,7 @@ constexpr int HT_ELE = 256;               // element places of a tile, at most (
 constexpr int HT_OWN = 170;               // owned nodes of a tile, at most
 constexpr int HT_NODES = 448;             // nodes staged per tile, at most
 constexpr int HT_ACC = HT_OWN * 3;        // sums of one wavefront
-constexpr int HT_LDS = HT_NODES * 6 + HT_THREADS / 64 * HT_ACC;  // values of LDS (37 KB in FP64)
+constexpr int HT_LDS = HT_NODES * 6 + HT_THREADS / 64 * HT_ACC;  // doubles of LDS (37 KB)
 
 // A tile owns up to HT_OWN nodes whose rows of K are sums of hex8 elements only and lists every
 // element incident to them, so the workgroup of a tile forms the whole product of its nodes: no
@@ -48,12 +48,18 @@ struct HexTilesHost {
     std::vector<int> nodes, rows, fams;
     std::vector<unsigned short> conn;
 };
-void hex_tiles_host(const Model &m, long long min_nodes, HexTilesHost &H);
+void hex_tiles_host(const Model &m, const std::vector<int> &nfe_off, const std::vector<int> &nfe_item, long long min_nodes,
+                    HexTilesHost &H);
 
 // Fewer nodes than this keep their rows in K: their tiles leave CUs idle through the several
 // microseconds of one tile (explicit step at 24^3 nodes: 8.5 us against 7.4 for the walk of K; at
 // 31^3: 11.8 against 13.0)
 constexpr long long HEX_MIN_NODES = 20480;
+// FP32 products walk the blocks up to this many nodes: 4-byte blocks stay in the 256 MB Infinity Cache
+// so long.  Explicit step: 31^3 nodes 9.5 us against 11.7 through the tiles; 60^3: 44.8 against 44.0,
+// for a longer first call; 66^3: 58.3 against 55.8; 80^3: 124 against 86.  Newmark iteration, penny
+// box: 48^3 107 against 110, 60^3 156 against 169, 80^3 409 against 349.
+constexpr int HEX_MIN_NODES_F32 = 262144;
 
 // The context's tiles (built on first use), or null where the products go through K: 2D models and
 // models with few nodes whose rows are hex8 sums (HEX_MIN_NODES)
@@ -61,9 +67,6 @@ int hex_tiles(Ctx &c, const HexTiles *&out, std::string &err);
 void free_hex_tiles(Ctx &c);
 
 // lane l ^ 1's value
-__device__ inline float pair_swap(float v) {
-    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xF, 0xF, true));
-}
 __device__ inline double pair_swap(double v) {
     const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), 0xB1, 0xF, 0xF, true);
     const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), 0xB1, 0xF, 0xF, true);
@@ -83,8 +86,13 @@ __device__ inline double pair_swap(double v) {
 // (J^-1 = A / det): G = A^T H, sigma = lam tr(G) I + mu (G + G^T) over det, P_k = A_k . sigma (detJ
 // cancels), then the transposes of the interpolations.  About 700 VALU instructions per thread.
 // MASS adds rho N_a N_b detJ of the consistent mass to the product (rho8 = rho / 8).
-template <typename T, bool MASS>
-__device__ inline void hex_plane(const T (&nb)[4][6], const T (&nt)[4][6], int h, T lam8, T mu8, T rho8, T (&f)[4][3]) {
+// FP64 for FP32 vectors too: without packed instructions FP32 arithmetic has FP64's rate, and the
+// FP32 form of this code took longer (115 us against 92 per product on the 80^3 box: its additions in
+// LDS, ds_add_f32, waited ten times as long).
+template <bool MASS>
+__device__ inline void hex_plane(const double (&nb)[4][6], const double (&nt)[4][6], int h, double lam8, double mu8,
+                                 double rho8, double (&f)[4][3]) {
+    using T = double;
     const T g0 = T(0.21132486540518711775), g1 = T(0.78867513459481288225);  // (1 -+ 1/sqrt 3) / 2
     const T mz = h ? g1 : g0;
     T s0[6], e0[6], cc[6], z0[6], zs[6], ze[6], zc[6], v0[3];
@@ -129,9 +137,7 @@ __device__ inline void hex_plane(const T (&nb)[4][6], const T (&nt)[4][6], int h
         }
         const T det = rx[0] * A0[0] + rx[1] * A0[1] + rx[2] * A0[2];
         // 1 / det: the hardware estimate and two Newton steps, within a unit in the last place
-        T inv;
-        if constexpr (sizeof(T) == 8) inv = __builtin_amdgcn_rcp(det);
-        else inv = __builtin_amdgcn_rcpf(det);
+        T inv = __builtin_amdgcn_rcp(det);
         inv = inv + inv * (T(1) - det * inv);
         inv = inv + inv * (T(1) - det * inv);
         T G[3][3];
@@ -189,8 +195,7 @@ __device__ inline void hex_plane(const T (&nb)[4][6], const T (&nt)[4][6], int h
 
 // addition to a sum in LDS in one operation (ds_add), and a point that the additions of a wavefront
 // are not moved across
-template <typename T>
-__device__ inline void lds_add(T *p, T v) {
+__device__ inline void lds_add(double *p, double v) {
     __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 __device__ inline void wave_order() {
@@ -205,9 +210,9 @@ __device__ inline void wave_order() {
 // are the same bits every time.  x is kept relative to a point of the tile, so that J does not lose
 // digits far from the origin.  Every thread of the workgroup must call it; after a barrier
 // hex_tile_sum(lds, n * 3 + c) is component c of owned node n and hex_tile_u(lds, n, c) its u.
-template <typename T, typename X, bool MASS>
+template <bool MASS, typename X>
 __device__ inline void hex_tile_product(const HexTile &t, const HexTiles &ht, const double *__restrict__ x,
-                                        const X *__restrict__ u, T lam8, T mu8, T rho8, T *lds) {
+                                        const X *__restrict__ u, double lam8, double mu8, double rho8, double *lds) {
     const int tid = threadIdx.x, wave = tid >> 6, h = tid & 1;
     // everything that depends on the tile alone is loaded before anything is waited for
     const uint4 *cn = reinterpret_cast<const uint4 *>(ht.conn) + t.ele0 + ((tid & 63) >> 1);
@@ -229,16 +234,16 @@ __device__ inline void hex_tile_product(const HexTile &t, const HexTiles &ht, co
                 uv[k][c] = u[o + c];
             }
         }
-    T *acc = lds + HT_NODES * 6 + wave * HT_ACC;
-    for (int k = tid & 63; k < t.n_own * 3; k += 64) acc[k] = T(0);
+    double *acc = lds + HT_NODES * 6 + wave * HT_ACC;
+    for (int k = tid & 63; k < t.n_own * 3; k += 64) acc[k] = 0.0;
 #pragma unroll
     for (int k = 0; k < NS; k++)
         if (id[k] >= 0) {
-            T *d = lds + (tid + k * HT_THREADS) * 6;
+            double *d = lds + (tid + k * HT_THREADS) * 6;
 #pragma unroll
             for (int c = 0; c < 3; c++) {
-                d[c] = T(xv[k][c] - t.x[c]);
-                d[3 + c] = T(uv[k][c]);
+                d[c] = xv[k][c] - t.x[c];
+                d[3 + c] = double(uv[k][c]);
             }
         }
     __syncthreads();
@@ -248,17 +253,17 @@ __device__ inline void hex_tile_product(const HexTile &t, const HexTiles &ht, co
         if ((g + HT_THREADS / 64) * HT_GROUP < t.n_ele) w = cn[(g + HT_THREADS / 64) * HT_GROUP];
         auto local = [&](int i) { return (l[i >> 1] >> (16 * (i & 1))) & 0xffffu; };
         if (local(0) == 0xffffu) continue;  // both threads of the pair
-        T nb[4][6], nt[4][6], f[4][3];
+        double nb[4][6], nt[4][6], f[4][3];
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            const T *b = lds + local(i) * 6, *a = lds + local(4 + i) * 6;
+            const double *b = lds + local(i) * 6, *a = lds + local(4 + i) * 6;
 #pragma unroll
             for (int c = 0; c < 6; c++) {
                 nb[i][c] = b[c];
                 nt[i][c] = a[c];
             }
         }
-        hex_plane<T, MASS>(nb, nt, h, lam8, mu8, rho8, f);
+        hex_plane<MASS>(nb, nt, h, lam8, mu8, rho8, f);
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             const int n = h ? local(4 + i) : local(i);
@@ -275,13 +280,9 @@ __device__ inline void hex_tile_product(const HexTile &t, const HexTiles &ht, co
     }
 }
 
-template <typename T>
-__device__ inline T hex_tile_u(const T *lds, int n, int c) {
-    return lds[n * 6 + 3 + c];
-}
-template <typename T>
-__device__ inline T hex_tile_sum(const T *lds, int k) {
-    T s = T(0);
+__device__ inline double hex_tile_u(const double *lds, int n, int c) { return lds[n * 6 + 3 + c]; }
+__device__ inline double hex_tile_sum(const double *lds, int k) {
+    double s = 0.0;
 #pragma unroll
     for (int w = 0; w < HT_THREADS / 64; w++) s += lds[HT_NODES * 6 + w * HT_ACC + k];
     return s;

@@ -29,6 +29,7 @@
 #include <numeric>
 
 #include "device.hpp"
+#include "hex.hpp"
 #include "reduce.hpp"
 #include "rowblock.hpp"
 
@@ -142,6 +143,62 @@ __global__ void __launch_bounds__(256) k_spmv_dot(const int *rows_s, int ns, int
     if (bp1) {
         d1 = block_sum(d1, sm);
         if (threadIdx.x == 0) bp1[slot] = d1;
+    }
+}
+
+// y = mask((ks K + ms M) x) with the same fused dots, most of the operator not read: the rows of the
+// hex8 nodes come from the elements, those of the interior PD nodes from their families' moments
+// (hex.hpp), the others from the operator's FP64 blocks K, a wavefront each.  FP64
+// arithmetic for FP32 vectors too.  Each block writes its dot partials to bp0 / bp1 at its own slot.
+// 80^3 penny box, K_eff: 92 us per product where the walk of its blocks takes 202 in FP64 and 120 in
+// FP32 (mirrored storage).  Bound as the explicit step's kernel is.
+template <typename V, bool MASS>
+__global__ void __launch_bounds__(HT_THREADS, HT_WAVES) k_spmv_hex(
+    HexTiles ht, MomentArgs ma, double ks, double lam8, double mu8, double rho8, double rho_pd, const int *adj_off, const int *adj,
+    const double *K, const double *xc, const V *x, V *y, const int *eq, const V *w0, double *bp0, const V *w1, double *bp1) {
+    __shared__ __align__(16) double lds[HT_LDS];
+    __shared__ double sm[17];
+    double d0 = 0.0, d1 = 0.0;
+    auto put = [&](size_t o, V v) {
+        const V yv = eq[o] >= 0 ? v : V(0);
+        y[o] = yv;
+        if (w0) d0 += double(w0[o]) * double(yv);
+        if (w1) d1 += double(w1[o]) * double(yv);
+    };
+    const HexTile t = ht.work[blockIdx.x];
+    if (t.n_own > 0) {
+        hex_tile_product<MASS>(t, ht, xc, x, lam8, mu8, rho8, lds);
+        __syncthreads();
+        for (int k = threadIdx.x; k < t.n_own * 3; k += HT_THREADS) {
+            const int n = k / 3;
+            put((size_t)ht.nodes[t.node0 + n] * 3 + (k - n * 3), V(hex_tile_sum(lds, k)));
+        }
+    } else if (t.n_own < 0) {
+        const int q = threadIdx.x / 16, lane = threadIdx.x % 16;
+        if (q < t.n_node) {
+            const int f = ht.fams[t.node0 + q];
+            double v[3];
+            family_row(ma, f, lane, xc, x, v);
+            if (lane < 3) {
+                const size_t o = (size_t)ma.fam_mem[ma.fam_off[f]] * 3 + lane;
+                put(o, V(ks * pick<3, double>(v, lane) + rho_pd * ma.fam_v[f] * double(x[o])));
+            }
+        }
+    } else {
+        const int q = threadIdx.x / 64;
+        if (q < t.n_node) {
+            const int r = ht.rows[t.node0 + q];
+            spmv_dot_row<3, double, V, 64, false, false, false>(r, adj_off, adj, nullptr, nullptr, nullptr, nullptr, K, nullptr,
+                                                                x, y, eq, w0, w1, d0, d1);
+        }
+    }
+    if (bp0) {
+        d0 = block_sum(d0, sm);
+        if (threadIdx.x == 0) bp0[blockIdx.x] = d0;
+    }
+    if (bp1) {
+        d1 = block_sum(d1, sm);
+        if (threadIdx.x == 0) bp1[blockIdx.x] = d1;
     }
 }
 
@@ -1059,14 +1116,24 @@ void free_two_level(Ctx &c) {
 // device pointers a captured chunk of iterations reads; a change of any of them re-captures
 struct GraphSig {
     const void *K = nullptr, *RS = nullptr, *tl = nullptr, *ilu = nullptr, *Pn = nullptr, *kp = nullptr,
-               *Ainv = nullptr, *rc = nullptr, *yc = nullptr, *red = nullptr, *src = nullptr;
+               *Ainv = nullptr, *rc = nullptr, *yc = nullptr, *red = nullptr, *src = nullptr, *ht = nullptr, *A64 = nullptr;
+    double ks = 0.0, ms = 0.0;
     long long K_gen = -1, tl_serial = -1, ilu_serial = -1;  // launch shapes follow these objects
     int krylov = -1;
     bool same(const GraphSig &o) const {
         return K == o.K && RS == o.RS && tl == o.tl && ilu == o.ilu && Pn == o.Pn && kp == o.kp && Ainv == o.Ainv &&
-               rc == o.rc && yc == o.yc && red == o.red && src == o.src && K_gen == o.K_gen && tl_serial == o.tl_serial &&
+               rc == o.rc && yc == o.yc && red == o.red && src == o.src && ht == o.ht && A64 == o.A64 && ks == o.ks && ms == o.ms && K_gen == o.K_gen && tl_serial == o.tl_serial &&
                ilu_serial == o.ilu_serial && krylov == o.krylov;
     }
+};
+
+// How a solve forms its products: the blocks K (own-index map src of mirrored storage or null) and, with
+// tiles, ks K + ms M through them
+struct Product {
+    const int *src = nullptr;
+    const HexTiles *ht = nullptr;
+    const double *A64 = nullptr;  // FP64 blocks for the rows outside the tiles
+    double ks = 0.0, ms = 0.0;
 };
 
 // Krylov workspace of one precision, kept on the context across solves so that the
@@ -1089,7 +1156,7 @@ struct KrylovWs {
     const float *Ainv32 = nullptr;  // the coarse inverse applied by both precisions
     const V *RS = nullptr;  // block row sums (difference-form SpMV) or null
     const void *ilu = nullptr;  // ILU(0) factor (ilu0.hip) or null
-    const int *src = nullptr;  // own index map when the iterations read mirrored storage, else null
+    Product op;  // how the iterations form their products
 };
 
 template <typename V>
@@ -1232,7 +1299,11 @@ static GraphSig make_sig(Ctx &c, const void *K, const KrylovWs<V> &w, int krylov
     g.rc = w.rc;
     g.yc = w.yc;
     g.red = c.red;
-    g.src = w.src;
+    g.src = w.op.src;
+    g.ht = w.op.ht;
+    g.A64 = w.op.A64;
+    g.ks = w.op.ks;
+    g.ms = w.op.ms;
     g.K_gen = c.K_gen;
     g.tl_serial = w.tl ? w.tl->serial : -1;
     g.ilu_serial = w.ilu ? ilu0_serial(w.ilu) : -1;
@@ -1246,9 +1317,23 @@ static GraphSig make_sig(Ctx &c, const void *K, const KrylovWs<V> &w, int krylov
 // per-block dot partials live in c.red after the RED_SLOTS partial slots (solve_masked allocates
 // them before any solve that asks for dots) and are folded by k_fold_parts.  Either way mirrored
 // and full storage run the same kernel, so their dots and results are the same bits.
+template <typename V>
+static void launch_spmv_hex(Ctx &c, const Product &P, const V *x, V *y, const V *w0, double *bp0, const V *w1,
+                            double *bp1) {
+    const double lam8 = P.ks * c.lambda / 8, mu8 = P.ks * c.mu / 8, rho8 = P.ms * c.rho / 8;
+#define PDX_SPMV_HEX(MASS)                                                                                        \
+    k_spmv_hex<V, MASS><<<P.ht->n_work, HT_THREADS, 0, c.stream>>>(                                               \
+        *P.ht, moment_args(c), P.ks, lam8, mu8, rho8, P.ms * c.rho, c.adj_off, c.adj, P.A64, c.x, x, y, c.eq, w0, bp0, w1, \
+        bp1)
+    if (P.ms != 0.0) PDX_SPMV_HEX(true);
+    else PDX_SPMV_HEX(false);
+#undef PDX_SPMV_HEX
+}
+
 template <int D, typename T, typename V>
-static void spmv_dot(Ctx &c, const T *K, const int *src, const T *RS, const V *x, V *y, const V *w0, double *p0,
+static void spmv_dot(Ctx &c, const T *K, const Product &P, const T *RS, const V *x, V *y, const V *w0, double *p0,
                      const V *w1, double *p1) {
+    const int *src = P.src;
     if constexpr (D < 3) {
 #define PDX_SPMV_DOT_P(REL, SYM)                                                                               \
     k_spmv_dot_p<D, T, V, REL, SYM><<<RED_PARTS, SPMV_THREADS, 0, c.stream>>>(                                \
@@ -1266,8 +1351,14 @@ static void spmv_dot(Ctx &c, const T *K, const int *src, const T *RS, const V *x
 #undef PDX_SPMV_DOT_P
     } else {
         const SpmvShape sh = spmv_shape(c);
+        const int grid = P.ht ? P.ht->n_work : sh.grid;
         double *bp = c.red ? c.red + (size_t)RED_SLOTS * NPART + 16 : nullptr;
-        double *bp0 = p0 ? bp : nullptr, *bp1 = p1 ? bp + sh.grid : nullptr;
+        double *bp0 = p0 ? bp : nullptr, *bp1 = p1 ? bp + grid : nullptr;
+        if (P.ht) {
+            launch_spmv_hex<V>(c, P, x, y, w0, bp0, w1, bp1);
+            if (p0 || p1) k_fold_parts<<<NPART, 64, 0, c.stream>>>(grid, bp0, p0, bp1, p1);
+            return;
+        }
         const int rev = int(c.spmv_calls++ & 1);  // every other product sweeps the rows in reverse
 #define PDX_SPMV_DOT(REL, SYM)                                                                                  \
     k_spmv_dot<D, T, V, REL, SYM><<<sh.grid, 256, 0, c.stream>>>(                                             \
@@ -1302,7 +1393,7 @@ static void bicg_iter(Ctx &c, const T *K, KrylovWs<V> &w, double *red, double *s
         k_coarse_mv<float><<<gc, 256, 0, c.stream>>>(t.nc, t.ld, w.Ainv32, w.rc, w.yc);
         k_prolong<D, NM, V><<<gn, 256, 0, c.stream>>>(c.nn, w.Pn, t.node_agg, t.kp_off, t.kp_agg, w.kp, w.Minv, w.p,
                                                       w.yc, w.ph);
-        spmv_dot<D, T, V>(c, K, w.src, (const T *)w.RS, w.ph, w.v, w.rh, rv, (const V *)nullptr, nullptr);
+        spmv_dot<D, T, V>(c, K, w.op, (const T *)w.RS, w.ph, w.v, w.rh, rv, (const V *)nullptr, nullptr);
         k_bicg_s_agg<D, NM, V><<<RED_PARTS, 256, 0, c.stream>>>(t.na, t.agg_off, t.agg_node, w.r, w.v, w.s, w.Pn,
                                                                 rho, rv, sc, w.rc);
         k_coarse_mv<float><<<gc, 256, 0, c.stream>>>(t.nc, t.ld, w.Ainv32, w.rc, w.yc);
@@ -1312,15 +1403,15 @@ static void bicg_iter(Ctx &c, const T *K, KrylovWs<V> &w, double *red, double *s
         k_bicg_p<D, V><<<RED_PARTS, 256, 0, c.stream>>>(c.nn, w.r, w.p, w.v, w.ph, (const V *)nullptr, rho, sc,
                                                         it == 0);
         ilu0_apply(c, w.ilu, w.p, w.ph);
-        spmv_dot<D, T, V>(c, K, w.src, (const T *)w.RS, w.ph, w.v, w.rh, rv, (const V *)nullptr, nullptr);
+        spmv_dot<D, T, V>(c, K, w.op, (const T *)w.RS, w.ph, w.v, w.rh, rv, (const V *)nullptr, nullptr);
         k_bicg_s<D, V><<<RED_PARTS, 256, 0, c.stream>>>(c.nn, w.r, w.v, w.s, w.sh, (const V *)nullptr, rho, rv, sc);
         ilu0_apply(c, w.ilu, w.s, w.sh);
     } else {
         k_bicg_p<D, V><<<RED_PARTS, 256, 0, c.stream>>>(c.nn, w.r, w.p, w.v, w.ph, w.Minv, rho, sc, it == 0);
-        spmv_dot<D, T, V>(c, K, w.src, (const T *)w.RS, w.ph, w.v, w.rh, rv, (const V *)nullptr, nullptr);
+        spmv_dot<D, T, V>(c, K, w.op, (const T *)w.RS, w.ph, w.v, w.rh, rv, (const V *)nullptr, nullptr);
         k_bicg_s<D, V><<<RED_PARTS, 256, 0, c.stream>>>(c.nn, w.r, w.v, w.s, w.sh, w.Minv, rho, rv, sc);
     }
-    spmv_dot<D, T, V>(c, K, w.src, (const T *)w.RS, w.sh, w.t, w.s, ts, w.t, tt);
+    spmv_dot<D, T, V>(c, K, w.op, (const T *)w.RS, w.sh, w.t, w.s, ts, w.t, tt);
     k_bicg_x<D, V><<<RED_PARTS, 256, 0, c.stream>>>(c.nn, w.x, w.r, w.rh, w.ph, w.sh, w.s, w.t, rho, ts, tt, sc,
                                                     rho_next, rr);
 }
@@ -1338,7 +1429,7 @@ static int bicgstab(Ctx &c, const T *K, KrylovWs<V> &w, const V *b, double bnorm
     double *y = w.y64;
     {
         V *tmp = w.t;
-        spmv_dot<D, T, V>(c, K, w.src, (const T *)w.RS, w.x, tmp, (const V *)nullptr, nullptr, (const V *)nullptr, nullptr);
+        spmv_dot<D, T, V>(c, K, w.op, (const T *)w.RS, w.x, tmp, (const V *)nullptr, nullptr, (const V *)nullptr, nullptr);
         k_copy<V, double><<<2048, 256, 0, c.stream>>>(n, tmp, y);
         k_resid<V, V><<<RED_PARTS, 256, 0, c.stream>>>(n, b, y, w.r, w.rh, red + (size_t)P_RR * NPART);
         k_dot<V><<<RED_PARTS, 256, 0, c.stream>>>(w.rh, w.r, n, red + (size_t)P_RHO0 * NPART);
@@ -1395,7 +1486,7 @@ static int pcg(Ctx &c, const T *K, KrylovWs<V> &w, const V *b, double bnorm, dou
     const size_t n = (size_t)c.nn * c.dim;
     double *red = c.red;
     double *y = w.y64;
-    spmv_dot<D, T, V>(c, K, w.src, (const T *)w.RS, w.x, w.t, (const V *)nullptr, nullptr, (const V *)nullptr, nullptr);
+    spmv_dot<D, T, V>(c, K, w.op, (const T *)w.RS, w.x, w.t, (const V *)nullptr, nullptr, (const V *)nullptr, nullptr);
     k_copy<V, double><<<2048, 256, 0, c.stream>>>(n, w.t, y);
     k_resid<V, V><<<RED_PARTS, 256, 0, c.stream>>>(n, b, y, w.r, nullptr, red + (size_t)P_RR * NPART);
     // z = Minv r and rho0 = (r, z) through a zero step
@@ -1417,7 +1508,7 @@ static int pcg(Ctx &c, const T *K, KrylovWs<V> &w, const V *b, double bnorm, dou
         double *rho_new = red + (size_t)((i & 1) ? P_RHO0 : P_RHO1) * NPART;
         double *rho_prev = rho_new;
         k_cg_p<V><<<RED_PARTS, 256, 0, c.stream>>>(n, w.p, w.s, rho, rho_prev, i == 0);
-        spmv_dot<D, T, V>(c, K, w.src, (const T *)w.RS, w.p, w.v, w.p, red + (size_t)P_RV * NPART, (const V *)nullptr,
+        spmv_dot<D, T, V>(c, K, w.op, (const T *)w.RS, w.p, w.v, w.p, red + (size_t)P_RV * NPART, (const V *)nullptr,
                           nullptr);
         k_cg_xr<D, V><<<RED_PARTS, 256, 0, c.stream>>>(c.nn, w.x, w.r, w.s, w.p, w.v, w.Minv, rho,
                                                       red + (size_t)P_RV * NPART, rho_new,
@@ -1525,6 +1616,33 @@ static int setup_precond(Ctx &c, const double *K64, const pdx_solve_opts &o, Kry
     return PDX_OK;
 }
 
+// the tiles that the products of a solve in precision prec with this context's operators go through (null:
+// the blocks; a solve whose FP32 products walk them forms its few FP64 residuals from them too)
+static int product_tiles(Ctx &c, int prec, const HexTiles *&ht, std::string &err) {
+    ht = nullptr;
+    if (c.dim != 3 || (prec == PDX_FP32 && c.nn < HEX_MIN_NODES_F32)) return PDX_OK;
+    if (int rc = hex_tiles(c, ht, err)) return rc;
+    return ht && ht->n_fam ? dev_family_moments(c, err) : PDX_OK;
+}
+
+int dev_product_tiles(Ctx &c, int prec, bool &tiles, std::string &err) {
+    const HexTiles *ht = nullptr;
+    const int rc = product_tiles(c, prec, ht, err);
+    tiles = ht;
+    return rc;
+}
+
+// y = mask(K x) in FP64 through the tiles (dev_product_tiles said so)
+int dev_spmv_tiles(Ctx &c, const double *x, double *y, std::string &err) {
+    Product P;
+    if (int rc = product_tiles(c, PDX_FP64, P.ht, err)) return rc;
+    P.A64 = c.K;
+    P.ks = 1.0;
+    launch_spmv_hex<double>(c, P, x, y, nullptr, nullptr, nullptr, nullptr);
+    PDX_HIP(hipGetLastError());
+    return PDX_OK;
+}
+
 // Solve K_ff x = b in FP64 (plain) or FP32 inner + FP64 refinement.
 // b_dev: full DOF vector (double, prescribed zero).  x_dev: in/out (double).
 // mir: own-block copies of the operator the SpMVs read instead of K64 / K32 (the
@@ -1534,11 +1652,35 @@ static int solve_masked(Ctx &c, const double *K64, const float *K32, const pdx_s
                         double *x_dev, pdx_solve_stats &st, std::string &err, const Mirrored &mir) {
     auto t0 = std::chrono::steady_clock::now();
     const size_t n = (size_t)c.nn * c.dim;
-    if (!c.red) {
-        // the partial slots, 16 scalars, then the SpMV's per-block partials of two dots
-        const size_t nred = (size_t)RED_SLOTS * NPART + 16 + 2 * (size_t)spmv_shape(c).grid;
+    // operator of the SpMVs: FP64 (residuals, FP64 iterations) and FP32 (FP32 iterations)
+    const int *src64 = D > 1 && mir.K64 ? c.ksrc : nullptr, *src32 = D > 1 && mir.K32 ? c.ksrc : nullptr;
+    const double *A64 = src64 ? mir.K64 : K64;
+    const float *A32 = src32 ? mir.K32 : K32;
+    Product op64, op32;
+    op64.src = src64;
+    op32.src = src32;
+    if (D == 3 && mir.ks != 0.0) {
+        if (int rc = product_tiles(c, o.precision, op64.ht, err)) return rc;
+        op64.A64 = K64;
+        op64.ks = mir.ks;
+        op64.ms = mir.ms;
+        if (op64.ht) {
+            op64.src = nullptr;
+            op32 = op64;
+        }
+    }
+    // the partial slots, 16 scalars, then the SpMV's per-block partials of two dots
+    const int blocks = std::max(spmv_shape(c).grid, op64.ht ? op64.ht->n_work : 0);
+    if (!c.red || c.red_blocks < blocks) {
+        if (c.red) {
+            PDX_HIP(hipStreamSynchronize(c.stream));
+            hipFree(c.red);
+            c.red = nullptr;
+        }
+        const size_t nred = (size_t)RED_SLOTS * NPART + 16 + 2 * (size_t)blocks;
         PDX_HIP(hipMalloc((void **)&c.red, sizeof(double) * nred));
         PDX_HIP(hipMemsetAsync(c.red, 0, sizeof(double) * nred, c.stream));
+        c.red_blocks = blocks;
     }
     double *part = c.red + (size_t)P_BB * NPART;
     k_dot<double><<<RED_PARTS, 256, 0, c.stream>>>(b_dev, b_dev, n, part);
@@ -1548,7 +1690,7 @@ static int solve_masked(Ctx &c, const double *K64, const float *K32, const pdx_s
     st.seconds = 0;
     st.true_relres = 1.0;
     st.converged = 0;
-    st.mirrored_used = D > 1 && mir.K64 && (o.precision == PDX_FP64 || mir.K32) ? 1 : 0;
+    st.mirrored_used = D > 1 && !op64.ht && mir.K64 && (o.precision == PDX_FP64 || mir.K32) ? 1 : 0;
     if (bnorm == 0.0) {
         PDX_HIP(hipMemsetAsync(x_dev, 0, n * 8, c.stream));
         PDX_HIP(hipStreamSynchronize(c.stream));
@@ -1563,15 +1705,11 @@ static int solve_masked(Ctx &c, const double *K64, const float *K32, const pdx_s
     if (!c.solve_y) PDX_HIP(hipMalloc((void **)&c.solve_y, n * 8));
     double *y = c.solve_y;
     const bool use_graph = !o.no_graph;
-    // operator of the SpMVs: FP64 (residuals, FP64 iterations) and FP32 (FP32 iterations)
-    const int *src64 = D > 1 && mir.K64 ? c.ksrc : nullptr, *src32 = D > 1 && mir.K32 ? c.ksrc : nullptr;
-    const double *A64 = src64 ? mir.K64 : K64;
-    const float *A32 = src32 ? mir.K32 : K32;
     if (o.precision == PDX_FP64) {
         KrylovWs<double> *wp;
         if ((rc = ws_get(c, wp, err)) || (rc = setup_precond<D, double>(c, K64, o, *wp, err))) return rc;
         KrylovWs<double> &w = *wp;
-        w.src = src64;
+        w.op = op64;
         PDX_HIP(hipMemcpyAsync(w.x, x_dev, n * 8, hipMemcpyDeviceToDevice, c.stream));
         double prev = INFINITY;
         for (int restart = 0; restart < 8; restart++) {
@@ -1584,7 +1722,7 @@ static int solve_masked(Ctx &c, const double *K64, const float *K32, const pdx_s
                                                    use_graph, &it, &rr, err);
             total += it;
             if (rc) break;
-            spmv_dot<D, double, double>(c, A64, src64, nullptr, w.x, y, (const double *)nullptr, nullptr,
+            spmv_dot<D, double, double>(c, A64, op64, nullptr, w.x, y, (const double *)nullptr, nullptr,
                                         (const double *)nullptr, nullptr);
             k_resid<double, double><<<RED_PARTS, 256, 0, c.stream>>>(n, b_dev, y, w.t, nullptr, part);
             rel = std::sqrt(host_sum(c, part, NPART, err)) / bnorm;
@@ -1593,22 +1731,24 @@ static int solve_masked(Ctx &c, const double *K64, const float *K32, const pdx_s
         }
         PDX_HIP(hipMemcpyAsync(x_dev, w.x, n * 8, hipMemcpyDeviceToDevice, c.stream));
     } else {
-        if (!K32) { err = "FP32 matrix missing"; return PDX_ERR_ARG; }
+        if (!K32 && !op32.ht) { err = "FP32 matrix missing"; return PDX_ERR_ARG; }
         KrylovWs<float> *wp;
         if (!c.solve_b32) PDX_HIP(hipMalloc((void **)&c.solve_b32, n * 4));
         float *b32 = c.solve_b32;
         if ((rc = ws_get(c, wp, err)) || (rc = setup_precond<D, float>(c, K64, o, *wp, err))) return rc;
         KrylovWs<float> &w = *wp;
-        w.src = src32;
-        if (!w.RSbuf) PDX_HIP(hipMalloc((void **)&w.RSbuf, (size_t)c.nn * c.dd * 4));
-        k_block_rowsum<D, float><<<(c.nn + 255) / 256, 256, 0, c.stream>>>(c.nn, c.adj_off, K64, w.RSbuf);
-        w.RS = w.RSbuf;
+        w.op = op32;
+        if (!op32.ht) {
+            if (!w.RSbuf) PDX_HIP(hipMalloc((void **)&w.RSbuf, (size_t)c.nn * c.dd * 4));
+            k_block_rowsum<D, float><<<(c.nn + 255) / 256, 256, 0, c.stream>>>(c.nn, c.adj_off, K64, w.RSbuf);
+            w.RS = w.RSbuf;
+        }
         const double inner = o.inner_tol > 0 ? o.inner_tol : 1e-4;
         double prev = INFINITY;
         int stalls = 0;
         for (refine = 0; refine < 60; refine++) {
             // FP64 residual r = b - K x
-            spmv_dot<D, double, double>(c, A64, src64, nullptr, x_dev, y, (const double *)nullptr, nullptr,
+            spmv_dot<D, double, double>(c, A64, op64, nullptr, x_dev, y, (const double *)nullptr, nullptr,
                                         (const double *)nullptr, nullptr);
             k_resid<float, double><<<RED_PARTS, 256, 0, c.stream>>>(n, b_dev, y, b32, nullptr, part);
             rel = std::sqrt(host_sum(c, part, NPART, err)) / bnorm;
@@ -1713,10 +1853,15 @@ int dev_solve(Ctx &c, const pdx_solve_opts &o, const double *b_dev, double *x_de
               std::string &err) {
     if (!c.K_valid) { err = "K not assembled"; return PDX_ERR_ARG; }
     int rc;
-    if (o.precision == PDX_FP32 && (rc = ensure_K32(c, err))) return rc;
+    bool tiles = false;
+    if ((rc = dev_product_tiles(c, o.precision, tiles, err))) return rc;
+    const bool walk32 = o.precision == PDX_FP32 && !tiles;
+    if (walk32 && (rc = ensure_K32(c, err))) return rc;
     Mirrored mir;
-    if (o.mirrored && c.dim > 1 && (rc = kown_for_solve(c, o.precision, mir, err))) return rc;
-    return dev_solve_mat(c, c.K, o.precision == PDX_FP32 ? c.K32 : nullptr, o, b_dev, x_dev, st, err, &mir);
+    // mirrored storage is for products that walk the blocks
+    if (o.mirrored && c.dim > 1 && !tiles && (rc = kown_for_solve(c, o.precision, mir, err))) return rc;
+    mir.ks = 1.0;
+    return dev_solve_mat(c, c.K, walk32 ? c.K32 : nullptr, o, b_dev, x_dev, st, err, &mir);
 }
 
 // ------------------------------------------------------------------------
@@ -1772,12 +1917,12 @@ static int probe_impl(Ctx &c, const double *K64, TwoLevel &t, const double *z, d
     for (int p = 0; p < nprobe; p++) {
         const double *zp = z + p * n;
         double *fp = f + p * n, *yp = y + p * n;
-        spmv_dot<D, double, double>(c, K64, nullptr, nullptr, zp, kz, (const double *)nullptr, nullptr, (const double *)nullptr,
+        spmv_dot<D, double, double>(c, K64, Product{}, nullptr, zp, kz, (const double *)nullptr, nullptr, (const double *)nullptr,
                                     nullptr);
         k_restrict_agg<D, NM><<<RED_PARTS, 256, 0, c.stream>>>(t.na, t.agg_off, t.agg_node, kz, t.Pn, rc);
         k_coarse_mv<double><<<gc, 256, 0, c.stream>>>(t.nc, t.ld, t.Ainv, rc, yc);
         k_sub_prolong<D, NM><<<(c.nn + 255) / 256, 256, 0, c.stream>>>(c.nn, t.Pn, t.node_agg, yc, zp, fp);
-        spmv_dot<D, double, double>(c, K64, nullptr, nullptr, fp, yp, (const double *)nullptr, nullptr, (const double *)nullptr,
+        spmv_dot<D, double, double>(c, K64, Product{}, nullptr, fp, yp, (const double *)nullptr, nullptr, (const double *)nullptr,
                                     nullptr);
     }
     PDX_HIP(hipGetLastError());

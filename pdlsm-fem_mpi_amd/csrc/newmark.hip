@@ -287,7 +287,10 @@ int dev_newmark(Ctx &c, int nsteps, const pdx_solve_opts &o, std::vector<double>
         if (rc && !o.fallback) return rc;
         rc = PDX_OK;
     }
-    if (o.precision == PDX_FP32) {
+    bool tiles = false;
+    if ((rc = dev_product_tiles(c, o.precision, tiles, err))) return rc;
+    const bool walk32 = o.precision == PDX_FP32 && !tiles;  // FP32 products walk the FP32 blocks
+    if (walk32) {
         rc = to_f32(c, Keff, Keff32, err);
         if (Keff32) owned.p.push_back(Keff32);
         if (rc) return rc;
@@ -295,15 +298,17 @@ int dev_newmark(Ctx &c, int nsteps, const pdx_solve_opts &o, std::vector<double>
     // mirrored storage of K_eff for the SpMVs, when its mirrored blocks are exact transposes
     // (K's are by construction; the consistent mass's are checked with them)
     Mirrored mir;
+    mir.ks = c.beta * c.dt * c.dt;
+    mir.ms = 1.0;
     double *own64 = nullptr;
     float *own32 = nullptr;
-    if (o.mirrored && c.dim > 1) {
+    if (o.mirrored && c.dim > 1 && !tiles) {
         bool exact = false;
         if ((rc = check_mirrored(c, Keff, exact, err))) return rc;
         if (exact) {
             const size_t no = (size_t)c.dd * std::max<long long>(c.n_own, 1);
             PDX_HIP(dalloc((void **)&own64, no * 8));
-            if (o.precision == PDX_FP32) PDX_HIP(dalloc((void **)&own32, no * 4));
+            if (walk32) PDX_HIP(dalloc((void **)&own32, no * 4));
             if ((rc = gather_own(c, Keff, own64, own32, err))) return rc;
             mir.K64 = own64;
             mir.K32 = own32;
@@ -345,7 +350,12 @@ int dev_newmark(Ctx &c, int nsteps, const pdx_solve_opts &o, std::vector<double>
         if (c.n_nbc) PDX_HIP(hipMemcpyAsync(nbcv_d, c.nbc_val.data(), c.n_nbc * 8, hipMemcpyHostToDevice, c.stream));
         k_predictor<<<(th + 255) / 256, 256, 0, c.stream>>>(c.nn, D, c.eq, c.presc_set, u, v, a, val, dU, c.dt,
                                                             c.beta, UN);
-        if ((rc = dev_spmv_K(c, c.K, UN, y))) { err = "spmv failed"; return rc; }
+        if (tiles) {
+            if ((rc = dev_spmv_tiles(c, UN, y, err))) return rc;
+        } else if ((rc = dev_spmv_K(c, c.K, UN, y))) {
+            err = "spmv failed";
+            return rc;
+        }
         k_newmark_rhs<<<(th + 255) / 256, 256, 0, c.stream>>>(th, y, c.f_unit, c.n_nbc, nbcv_d, c.eq, D, F);
         // initial guess a_{n+1} <- a_n (warm start), or 2 a_n - a_{n-1} (warm_start 2, from the
         // second step on)
@@ -393,7 +403,7 @@ int dev_newmark(Ctx &c, int nsteps, const pdx_solve_opts &o, std::vector<double>
                     if (rc && !o.fallback) break;
                     rc = PDX_OK;
                 }
-                if (o.precision == PDX_FP32 && (rc = to_f32(c, Keff, Keff32, err))) break;
+                if (walk32 && (rc = to_f32(c, Keff, Keff32, err))) break;
                 if (mir.K64 && (rc = gather_own(c, Keff, own64, own32, err))) break;
             }
         }

@@ -132,9 +132,9 @@ __global__ void __launch_bounds__(256) k_explicit(const int *rows_s, int ns, int
 // FP32: K is 330 MB (196 MB) per step there, while the elements are 8.6M FP64 wavefront instructions (15 us at the full rate) on some 60 MB.  Bound by
 // those two one after the other: two workgroups of 198 registers fit a CU, and the ones in flight load
 // together and calculate together.
-template <typename T, bool FO>
+template <bool FO>
 __global__ void __launch_bounds__(HT_THREADS, HT_WAVES) k_explicit_hex(
-    HexTiles ht, MomentArgs ma, double lam8, double mu8, const int *adj_off, const int *adj, const T *K,
+    HexTiles ht, MomentArgs ma, double lam8, double mu8, const int *adj_off, const int *adj, const double *K,
     const double *x, const double *Un, const double *Unm1, double *Unp1, const double *m, const double *f_unit, int n_nbc,
     int nn, const double *nbc_cur, double *nbc_next, const double *nbc_inc, const int *eq, const int *presc_set,
     const double *ebc_inc, double dt, int startup) {
@@ -168,7 +168,7 @@ __global__ void __launch_bounds__(HT_THREADS, HT_WAVES) k_explicit_hex(
     };
     const HexTile t = ht.work[blockIdx.x];
     if (t.n_own > 0) {
-        hex_tile_product<double, double, false>(t, ht, x, Un, lam8, mu8, 0.0, lds);
+        hex_tile_product<false>(t, ht, x, Un, lam8, mu8, 0.0, lds);
         // the owned DOFs' state is on its way while the last wavefronts still add
         constexpr int ND = (HT_OWN * 3 + HT_THREADS - 1) / HT_THREADS;
         Dof d[ND];
@@ -199,9 +199,9 @@ __global__ void __launch_bounds__(HT_THREADS, HT_WAVES) k_explicit_hex(
         const int row = ht.rows[t.node0 + q];
         Dof d;
         if (lane < 3) d = load(row, lane);
-        T acc[3];
-        row_matvec<3, T, double, 64, sizeof(T) == 4>(row, lane, adj_off, adj, K, Un, acc);
-        if (lane < 3) update(d, Un[d.o], double(pick<3, T>(acc, lane)));
+        double acc[3];
+        row_matvec<3, double, double, 64, false>(row, lane, adj_off, adj, K, Un, acc);
+        if (lane < 3) update(d, Un[d.o], pick<3, double>(acc, lane));
     }
 }
 
@@ -455,11 +455,6 @@ static void launch_explicit_any(Ctx &c, int prec, int variant, const double *Un,
     }
 }
 
-// FP32 steps walk K up to this many nodes: its 4-byte values stay in the 256 MB Infinity Cache so
-// long (31^3 nodes: 9.5 us against 11.7 through the tiles; 60^3: 44.8 against 44.0, for a longer
-// first call; 66^3: 58.3 against 55.8; 80^3: 124 against 86)
-constexpr int HEX_MIN_NODES_F32 = 262144;
-
 // the tiles a step of precision index pi goes through, or null when it walks K in one of the forms
 // (a form set by the caller, or no tiles for this model)
 static int step_tiles(Ctx &c, int pi, const HexTiles *&ht, std::string &err) {
@@ -468,11 +463,11 @@ static int step_tiles(Ctx &c, int pi, const HexTiles *&ht, std::string &err) {
     return hex_tiles(c, ht, err);
 }
 
-template <typename T, bool FO>
-static void launch_explicit_hex(Ctx &c, const HexTiles &ht, const T *K, const double *Un, const double *Unm1,
-                                double *Unp1, const double *nbc_cur, double *nbc_next, int startup) {
-    k_explicit_hex<T, FO><<<ht.n_work, HT_THREADS, 0, c.stream>>>(
-        ht, moment_args(c), c.lambda / 8, c.mu / 8, c.adj_off, c.adj, K, c.x, Un, Unm1, Unp1, c.mlump, c.f_unit, c.n_nbc, c.nn,
+template <bool FO>
+static void launch_explicit_hex(Ctx &c, const HexTiles &ht, const double *Un, const double *Unm1, double *Unp1,
+                                const double *nbc_cur, double *nbc_next, int startup) {
+    k_explicit_hex<FO><<<ht.n_work, HT_THREADS, 0, c.stream>>>(
+        ht, moment_args(c), c.lambda / 8, c.mu / 8, c.adj_off, c.adj, c.K, c.x, Un, Unm1, Unp1, c.mlump, c.f_unit, c.n_nbc, c.nn,
         nbc_cur, nbc_next, c.d_nbc_vel, c.eq, c.presc_set, c.d_ebc_vel, c.dt, startup);
 }
 
@@ -521,10 +516,8 @@ static void explicit_step(Ctx &c, int prec, int startup) {
     const HexTiles *ht = nullptr;
     std::string unused;  // the tiles, if any, were built by explicit_operators
     step_tiles(c, prec == PDX_FP32 ? 1 : 0, ht, unused);
-    if (ht && prec == PDX_FP32)
-        launch_explicit_hex<float, false>(c, *ht, c.K32, Un, Unm1, Unp1, nbc_cur, nbc_next, startup);
-    else if (ht)
-        launch_explicit_hex<double, false>(c, *ht, c.K, Un, Unm1, Unp1, nbc_cur, nbc_next, startup);
+    if (ht)
+        launch_explicit_hex<false>(c, *ht, Un, Unm1, Unp1, nbc_cur, nbc_next, startup);
     else
         launch_explicit_any(c, prec, std::max(c.tune_explicit[prec == PDX_FP32 ? 1 : 0], 0), Un, Unm1, Unp1, nbc_cur,
                             nbc_next, startup, s);
@@ -597,12 +590,13 @@ static int explicit_operators(Ctx &c, int prec, bool lumped, std::string &err) {
         int e = dev_assemble_K(c, err);
         if (e) return e;
     }
-    if (prec == PDX_FP32) {
+    const HexTiles *ht = nullptr;
+    if (lumped)
+        if (int e = step_tiles(c, prec == PDX_FP32 ? 1 : 0, ht, err)) return e;
+    if (prec == PDX_FP32 && !ht) {
         int e = ensure_K32(c, err);
         if (e) return e;
     }
-    const HexTiles *ht = nullptr;
-    if (int e = step_tiles(c, prec == PDX_FP32 ? 1 : 0, ht, err)) return e;
     if (ht) {
         if (ht->n_fam)
             if (int e = dev_family_moments(c, err)) return e;
@@ -698,8 +692,10 @@ int explicit_tune_if_needed(Ctx &c, int prec, std::string &err) {
 int explicit_tune_seen(Ctx &c, int pi, std::string &err) {
     if (c.tune_explicit[pi] >= 0 || c.tune_seen[pi] >= 0 || !c.hex || c.steps_done < 0) return PDX_OK;
     const int prec = pi ? PDX_FP32 : PDX_FP64;
-    if (!c.K_valid || (pi && !c.K32_valid)) return PDX_OK;
+    if (!c.K_valid) return PDX_OK;
     int rc;
+    if (!c.mlump_valid && (rc = dev_lumped_mass(c, err))) return rc;
+    if (pi && (rc = ensure_K32(c, err))) return rc;
     if ((rc = ensure_Ks(c, prec, err)) || (rc = ensure_Kown(c, prec, err)) || (rc = tune_explicit(c, pi, err))) return rc;
     c.tune_seen[pi] = c.tune_explicit[pi];
     c.tune_explicit[pi] = -1;

@@ -1,4 +1,5 @@
-"""The products with hex8 elements and PD families without their blocks of K (csrc/hex.hip) against the walk of K.
+"""The products with hex8 elements and PD families without their blocks of K (csrc/hex.hip) against the walk of K
+(explicit steps) and against the assembled K and mass on the host (solves).
 
 Both sum the same terms in FP64 in another order, so a trajectory differs by rounding only: a product of a row of some
 30 to 130 blocks of 3 x 3 carries at most about 400 roundings of 1.1e-16 of its absolute terms, 5e-14, and the
@@ -96,3 +97,48 @@ def test_fp32_force_through_tiles():
     e_tiles = rel(tiles.explicit_run(25, pdx.PDX_FP32)[0], u)
     e_walk = rel(walk.explicit_run(25, pdx.PDX_FP32)[0], u)
     assert e_tiles <= 1.2 * e_walk <= 1e-6
+
+
+def _csr(model, values):
+    import scipy.sparse as sp
+    ia, ja = model.csr()
+    return sp.csr_matrix((values, ja, ia), shape=(model.neq, model.neq))
+
+
+SOLVES = {"fp64": {}, "fp64_mirrored": {"mirrored": True}, "fp64_two_level": {"precond": 4}, "fp32_two_level": {"precision": 1, "precond": 4}}
+
+
+@pytest.mark.parametrize("opts", list(SOLVES))
+@pytest.mark.parametrize("name", list(CASES))
+def test_solves_through_tiles(name, opts):
+    """A Newmark step and a static solve: the residual of their results with the assembled matrices on the host, which
+    the solver's own products come within rounding of (1e-8 asked for; 1e-11 for the products' rounding)."""
+    mesh = _dt(CASES[name]())
+    mesh["nbc"][0]["val"] = 1e6
+    model = pdx.Model(mesh)
+    cx = pdx.Context(model)
+    K = _csr(model, cx.assemble(pdx.PDX_MODE_STATIC)[0])
+    o = dict(precond=pdx.PDX_PREC_BLOCK_JACOBI, tol=1e-8)
+    o.update(SOLVES[opts])
+    _, _, a, st = cx.newmark_run(1, pdx.solve_opts(**o))
+    keff = _csr(model, cx.mass_on_K()) + mesh["beta"] * mesh["dt"] ** 2 * K
+    dU = model.values()  # u = v = a = 0: the predictor is the prescribed values, advanced
+    for s in mesh["ebc"]:
+        dU[(np.asarray(s["nid"]) - 1) * 3 + s["dof"]] += mesh["dt"] * s.get("vel", 0.0) * bool(s.get("vary", False))
+    fresh = pdx.Context(model)
+    F = fresh.assemble(pdx.PDX_MODE_NEWMARK, UN=dU)[1]
+    assert np.linalg.norm(F - keff @ a) <= (1e-8 + 1e-11) * np.linalg.norm(F)
+    assert st["converged"]
+    u, st = fresh.static_solve(pdx.solve_opts(**o))
+    b = fresh.assemble(pdx.PDX_MODE_STATIC)[1]
+    assert np.linalg.norm(b - K @ u) <= (1e-8 + 1e-11) * np.linalg.norm(b)
+
+
+def test_fp32_newmark_through_tiles():
+    """FP32 vectors with FP64 element arithmetic (large models only), refined: the same displacements as in FP64."""
+    model = pdx.Model(_dt(W.box3d(n=65, pd_block=12)))
+    run = [pdx.Context(model).newmark_run(2, pdx.solve_opts(precond=pdx.PDX_PREC_BLOCK_JACOBI, precision=p, tol=1e-10))
+           for p in (pdx.PDX_FP64, pdx.PDX_FP32)]
+    assert run[1][3]["converged"] and run[1][3]["refinements"] > 0
+    for x, y in zip(run[0][:3], run[1][:3]):
+        assert rel(y, x) <= 1e-8
