@@ -28,6 +28,7 @@
 
 #include "../../include/pdx.h"
 #include "device.hpp"
+#include "normals.hpp"
 #include "reduce.hpp"
 
 namespace pdx {
@@ -540,14 +541,10 @@ static int gnn_probes(Ctx &c, GnnWork &g, int P, unsigned long long seed, int ag
     }
     const Model &m = *c.host;
     std::vector<double> z(P * n, 0.0);
-    std::mt19937_64 rng(seed);
-    std::normal_distribution<double> nd(0.0, 1.0);
-    for (int p = 0; p < P; p++)
-        for (int a = 0; a < g.nn; a++)
-            for (int i = 0; i < g.D; i++) {
-                const double v = nd(rng);
-                if (m.eq[(size_t)a * 3 + i] >= 0) z[p * n + (size_t)a * g.D + i] = v;
-            }
+    seeded_normals(seed, P * n, [&](size_t i, double v) {
+        const size_t q = i % n, a = q / g.D;
+        if (m.eq[a * 3 + (q - a * g.D)] >= 0) z[i] = v;
+    });
     double *zd, *fd, *yd;
     PDX_HIP(hipMalloc((void **)&zd, P * n * 8));
     PDX_HIP(hipMalloc((void **)&fd, P * n * 8));
