@@ -686,57 +686,110 @@ __global__ void k_blockjacobi(int nn, const int *adj_off, const int *adj, const 
 // ------------------------------------------------------------------------
 // A P on every node row: kp[q] (D x NM) for the q-th aggregate touched by row a
 // (rows of prescribed DOFs zero, since the operator is masked)
+// One lane per (row i of the node, mode m): it walks the node's blocks in order and adds K_ab P_b to the sum of
+// the block's aggregate in LDS (CAP aggregates at a time).  A thread per node that walked its row once per
+// aggregate took 736 us on the 41^3 box, this form 200 us.
 template <int D, int NM>
-__global__ void k_coarse_ap(int nn, const int *adj_off, const int *adj, const double *K, const double *Pn,
-                            const int *blk_slot, const int *kp_off, const int *eq, double *kp) {
-    const int a = blockIdx.x * blockDim.x + threadIdx.x;
-    if (a >= nn) return;
-    for (int q = kp_off[a]; q < kp_off[a + 1]; q++) {
-        const int slot = q - kp_off[a];
-        double s[D * NM];
+constexpr int AP_NODES = 252 / (D * NM);  // nodes of a 256-thread block
+template <int D, int NM>
+__global__ void __launch_bounds__(256) k_coarse_ap(int nn, const int *adj_off, const int *adj, const double *K,
+                                                   const double *Pn, const int *blk_slot, const int *kp_off,
+                                                   const int *eq, double *kp) {
+    constexpr int E = D * NM, CAP = D == 3 ? 16 : 8;
+    __shared__ double acc[AP_NODES<D, NM>][CAP][E];
+    const int g = threadIdx.x / E, e = threadIdx.x % E, i = e / NM, m = e % NM;
+    const int a = blockIdx.x * AP_NODES<D, NM> + g;
+    if (g >= AP_NODES<D, NM> || a >= nn) return;
+    const int q0 = kp_off[a], ns = kp_off[a + 1] - q0, b0 = adj_off[a], b1 = adj_off[a + 1];
+    const bool fr = eq[a * 3 + i] >= 0;
+    for (int s0 = 0; s0 < ns; s0 += CAP) {
+        const int cnt = min(CAP, ns - s0);
+        for (int k = 0; k < cnt; k++) acc[g][k][e] = 0.0;
+#pragma unroll 4
+        for (int b = b0; b < b1; b++) {
+            const int sl = blk_slot[b] - s0, c = adj[b];
+            double kv[D], pv[D];
 #pragma unroll
-        for (int e = 0; e < D * NM; e++) s[e] = 0.0;
-        for (int b = adj_off[a]; b < adj_off[a + 1]; b++) {
-            if (blk_slot[b] != slot) continue;
-            const int c = adj[b];
+            for (int j = 0; j < D; j++) {
+                kv[j] = K[(size_t)b * D * D + i * D + j];
+                pv[j] = Pn[((size_t)c * D + j) * NM + m];
+            }
+            if (sl < 0 || sl >= CAP) continue;
+            double s = acc[g][sl][e];
 #pragma unroll
-            for (int i = 0; i < D; i++)
-#pragma unroll
-                for (int j = 0; j < D; j++) {
-                    const double k = K[(size_t)b * D * D + i * D + j];
-#pragma unroll
-                    for (int m = 0; m < NM; m++) s[i * NM + m] += k * Pn[((size_t)c * D + j) * NM + m];
-                }
+            for (int j = 0; j < D; j++) s += kv[j] * pv[j];
+            acc[g][sl][e] = s;
         }
-#pragma unroll
-        for (int i = 0; i < D; i++) {
-            const bool fr = eq[a * 3 + i] >= 0;
-#pragma unroll
-            for (int m = 0; m < NM; m++) kp[((size_t)q * D + i) * NM + m] = fr ? s[i * NM + m] : 0.0;
-        }
+        for (int k = 0; k < cnt; k++) kp[(size_t)(q0 + s0 + k) * E + e] = fr ? acc[g][k][e] : 0.0;
     }
 }
 
-// dense Galerkin matrix: one thread per coarse row (I, m); Ac[row][J*NM+m'] += P_a^T (A P)_aJ
+// Dense Galerkin matrix: a workgroup per aggregate I forms its NM rows; Ac[row][J*NM+m'] += P_a^T (A P)_aJ over
+// its nodes a in order.  The aggregates J that its nodes reach are listed first (a bit each in LDS), then
+// every thread owns one value (J, m, m') and walks the nodes' lists, staged in LDS 256 nodes at a time.
+// One thread per coarse row, adding to memory, took 1,940 us on the 41^3 box, this form 235 us (501x251
+// plate: 285 and 179 us).
 template <int D, int NM>
-__global__ void k_coarse_galerkin(int na, const int *agg_off, const int *agg_node, const double *Pn,
-                                  const int *kp_off, const int *kp_agg, const double *kp, int ld, double *Ac) {
-    const int row = blockIdx.x * blockDim.x + threadIdx.x;
-    if (row >= na * NM) return;
-    const int I = row / NM, m = row % NM;
-    double *out = Ac + (size_t)row * ld;
-    for (int q0 = agg_off[I]; q0 < agg_off[I + 1]; q0++) {
-        const int a = agg_node[q0];
+__global__ void __launch_bounds__(1024) k_coarse_galerkin(int na, const int *agg_off, const int *agg_node,
+                                                          const double *Pn, const int *kp_off, const int *kp_agg,
+                                                          const double *kp, int ld, double *Ac) {
+    extern __shared__ unsigned gbits[];  // [(na + 31) / 32]
+    constexpr int JM = 512, NC = 256, LJ = 8;
+    __shared__ int jl[JM], njs, node[NC], first[NC], count[NC], lj[NC][LJ];
+    const int I = blockIdx.x, t = threadIdx.x, words = (na + 31) / 32;
+    const int n0 = agg_off[I], n1 = agg_off[I + 1];
+    for (int w = t; w < words; w += blockDim.x) gbits[w] = 0;
+    __syncthreads();
+    for (int n = n0 + t; n < n1; n += blockDim.x) {
+        const int a = agg_node[n];
         for (int q = kp_off[a]; q < kp_off[a + 1]; q++) {
             const int J = kp_agg[q];
-#pragma unroll
-            for (int m2 = 0; m2 < NM; m2++) {
-                double s = 0.0;
-#pragma unroll
-                for (int i = 0; i < D; i++) s += Pn[((size_t)a * D + i) * NM + m] * kp[((size_t)q * D + i) * NM + m2];
-                out[(size_t)J * NM + m2] += s;
-            }
+            atomicOr(&gbits[J >> 5], 1u << (J & 31));
         }
+    }
+    for (int done = 0;;) {  // JM aggregates at a time
+        __syncthreads();
+        if (t == 0) {
+            int n = 0;
+            for (int w = done; w < words && n + 32 <= JM; done = ++w)
+                for (unsigned v = gbits[w]; v; v &= v - 1) jl[n++] = w * 32 + __ffs(v) - 1;
+            njs = n;
+            jl[JM - 1] = done;  // the list is never that long: the next word to look at
+        }
+        __syncthreads();
+        const int nj = njs;
+        done = jl[JM - 1];
+        for (int v0 = 0; v0 < nj * NM * NM; v0 += blockDim.x) {
+            const int v = v0 + t, e = v % (NM * NM), m = e / NM, m2 = e % NM;
+            const int J = v < nj * NM * NM ? jl[v / (NM * NM)] : -1;
+            double out = 0.0;
+            for (int c0 = n0; c0 < n1; c0 += NC) {
+                // the chunk's nodes and the first LJ entries of their lists
+                __syncthreads();
+                const int nc = min(NC, n1 - c0);
+                if (t < nc) {
+                    const int a = agg_node[c0 + t], q0 = kp_off[a], cnt = kp_off[a + 1] - q0;
+                    node[t] = a;
+                    first[t] = q0;
+                    count[t] = cnt;
+                    for (int k = 0; k < min(cnt, LJ); k++) lj[t][k] = kp_agg[q0 + k];
+                }
+                __syncthreads();
+                for (int n = 0; n < nc; n++) {
+                    const int cnt = count[n];
+                    for (int k = 0; k < cnt; k++) {
+                        if ((k < LJ ? lj[n][k] : kp_agg[first[n] + k]) != J) continue;
+                        const int a = node[n], q = first[n] + k;
+                        double s = 0.0;
+#pragma unroll
+                        for (int i = 0; i < D; i++) s += Pn[((size_t)a * D + i) * NM + m] * kp[((size_t)q * D + i) * NM + m2];
+                        out += s;
+                    }
+                }
+            }
+            if (J >= 0) Ac[((size_t)I * NM + m) * ld + (size_t)J * NM + m2] = out;
+        }
+        if (done >= words) break;
     }
 }
 
@@ -750,113 +803,211 @@ __global__ void k_diag_copy(int n, int ld, const double *A, double *d) {
 // symmetric part; a pivot below 1e-12 of the DOF's original diagonal marks a
 // coarse mode without support (e.g. a rotation of a one-node aggregate): its
 // row and column are removed (zero in the inverse).
-constexpr int GJB = 64;
+constexpr int GJB = 64;    // pivot block and tile edge
+constexpr int GJP = 128;   // pivots per pass over the matrix: two blocks
 
-__global__ void __launch_bounds__(1024) k_gj_diag(int ld, int k, const double *A, const double *diag0, double *Dk) {
-    __shared__ double S[GJB][GJB + 1];
-    __shared__ double colq[GJB];
-    const int t = threadIdx.x, base = k * GJB, nt = blockDim.x;
-    for (int e = t; e < GJB * GJB; e += nt) S[e / GJB][e % GJB] = A[(size_t)(base + e / GJB) * ld + base + e % GJB];
+// Dk = inverse of a pivot block, in registers: wavefront w holds columns 16 w ... 16 w + 15, lane l row l.
+// Per pivot q the wavefront that owns column q passes it through LDS (two buffers, one barrier), row q
+// comes from lane q of each wavefront's own registers.  Bound by the issue of a pivot's 150 instructions,
+// one wavefront to a SIMD: the block in LDS with five barriers per pivot took 80 us, 16 wavefronts of 4
+// columns 56, this form 29 (the same operations on every entry, so the same bits).
+__global__ void __launch_bounds__(256) k_gj_diag(const double *A, int ld, const double *diag0, double *Dk) {
+    __shared__ double col[2][GJB], d0[GJB];
+    const int t = threadIdx.x, w = t >> 6, l = t & 63;
+    if (t < GJB) d0[t] = diag0[t];
+    double S[16];
+#pragma unroll
+    for (int j = 0; j < 16; j++) S[j] = A[(size_t)l * ld + 16 * w + j];
     __syncthreads();
-    for (int q = 0; q < GJB; q++) {
-        const double piv = S[q][q];
-        const double d0 = diag0[base + q];
-        const bool dropq = !(fabs(piv) > 1e-12 * fabs(d0)) || d0 == 0.0;
-        if (t < GJB) colq[t] = S[t][q];
-        __syncthreads();
-        if (dropq) {
-            if (t < GJB) { S[q][t] = 0.0; S[t][q] = 0.0; }
+    for (int own = 0; own < 4; own++) {
+#pragma unroll
+        for (int j = 0; j < 16; j++) {
+            const int q = 16 * own + j;
+            double *cb = col[j & 1];
+            if (w == own) cb[l] = S[j];
             __syncthreads();
-            continue;
+            const double piv = cb[q], ci = cb[l], dq = d0[q];
+            const bool dropq = !(fabs(piv) > 1e-12 * fabs(dq)) || dq == 0.0;
+            if (dropq) {  // row and column q out of the inverse
+#pragma unroll
+                for (int jj = 0; jj < 16; jj++)
+                    if (l == q) S[jj] = 0.0;
+                if (w == own) S[j] = 0.0;
+                continue;
+            }
+            const double ip = 1.0 / piv;
+#pragma unroll
+            for (int jj = 0; jj < 16; jj++) {
+                const double r = __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(S[jj]), q),
+                                                  __builtin_amdgcn_readlane(__double2loint(S[jj]), q)) * ip;
+                S[jj] = l == q ? r : S[jj] - ci * r;
+            }
+            if (w == own) S[j] = l == q ? ip : -ci * ip;
         }
-        const double ip = 1.0 / piv;
-        if (t < GJB && t != q) S[q][t] *= ip;
-        __syncthreads();
-        for (int e = t; e < GJB * GJB; e += nt) {
-            const int i = e / GJB, j = e % GJB;
-            if (i == q) continue;
-            if (j == q) S[i][j] = -colq[i] * ip;
-            else S[i][j] -= colq[i] * S[q][j];
-        }
-        __syncthreads();
-        if (t == 0) S[q][q] = ip;
-        __syncthreads();
     }
-    for (int e = t; e < GJB * GJB; e += nt) Dk[e] = S[e / GJB][e % GJB];
+#pragma unroll
+    for (int j = 0; j < 16; j++) Dk[l * GJB + 16 * w + j] = S[j];
 }
 
 typedef double gj_d4 __attribute__((ext_vector_type(4)));
 
-// C = alpha * A_blk * B_blk (+ C when acc): 64 x 64 tiles through LDS; each of the 4
-// waves computes a 32 x 32 quadrant as 2 x 2 tiles of v_mfma_f64_16x16x4f64 (operand lane l:
-// A[i = l%16][k = l/16], B[k = l/16][j = l%16]; result lane l item r: row l/16 + 4 r, col l%16)
-__device__ inline void tile_mm(const double *A, int lda, const double *B, int ldb, double *C, int ldc, double alpha,
-                               bool acc, double (*As)[GJB + 1], double (*Bs)[GJB + 1]) {
-    const int t = threadIdx.x;
-    for (int e = t; e < GJB * GJB; e += 256) {
-        As[e / GJB][e % GJB] = A[(size_t)(e / GJB) * lda + e % GJB];
-        Bs[e / GJB][e % GJB] = B[(size_t)(e / GJB) * ldb + e % GJB];
+// c = A B for 64 x 64 tiles through LDS; each of the 4 waves computes a 32 x 32 quadrant as 2 x 2 tiles of
+// v_mfma_f64_16x16x4f64 (operand lane l: A[i = l%16][k = l/16], B[k = l/16][j = l%16]; result lane l
+// item r: row l/16 + 4 r, col l%16)
+struct GjTile {
+    gj_d4 c[2][2];
+    // f(row, column, value) for this thread's entries
+    template <typename F>
+    __device__ void each(F &&f) const {
+        const int t = threadIdx.x, w = t >> 6, l = t & 63, row = (w >> 1) * 32 + (l >> 4), colm = (w & 1) * 32 + (l & 15);
+#pragma unroll
+        for (int a = 0; a < 2; a++)
+#pragma unroll
+            for (int b = 0; b < 2; b++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) f(row + 16 * a + 4 * r, colm + 16 * b, c[a][b][r]);
     }
-    __syncthreads();
-    const int w = t >> 6, l = t & 63;
+};
+struct GjLoad {  // a thread's share of two operand tiles, on its way to LDS
+    double a[16], b[16];
+    __device__ GjLoad(const double *A, int lda, const double *B, int ldb) {
+#pragma unroll
+        for (int n = 0; n < 16; n++) {
+            const int e = threadIdx.x + 256 * n;
+            a[n] = A[(size_t)(e / GJB) * lda + e % GJB];
+            b[n] = B[(size_t)(e / GJB) * ldb + e % GJB];
+        }
+    }
+    __device__ void store(double (*As)[GJB + 1], double (*Bs)[GJB + 1]) const {
+#pragma unroll
+        for (int n = 0; n < 16; n++) {
+            const int e = threadIdx.x + 256 * n;
+            As[e / GJB][e % GJB] = a[n];
+            Bs[e / GJB][e % GJB] = b[n];
+        }
+    }
+};
+__device__ inline GjTile gj_product(double (*As)[GJB + 1], double (*Bs)[GJB + 1]) {
+    const int t = threadIdx.x, w = t >> 6, l = t & 63;
     const int wr = (w >> 1) * 32, wc = (w & 1) * 32, li = l & 15, lk = l >> 4;
-    gj_d4 c00 = {0, 0, 0, 0}, c01 = {0, 0, 0, 0}, c10 = {0, 0, 0, 0}, c11 = {0, 0, 0, 0};
+    GjTile T = {};
     for (int k0 = 0; k0 < GJB; k0 += 4) {
         const int kk = k0 + lk;
         const double a0 = As[wr + li][kk], a1 = As[wr + 16 + li][kk];
         const double b0 = Bs[kk][wc + li], b1 = Bs[kk][wc + 16 + li];
-        c00 = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b0, c00, 0, 0, 0);
-        c01 = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b1, c01, 0, 0, 0);
-        c10 = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b0, c10, 0, 0, 0);
-        c11 = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b1, c11, 0, 0, 0);
+        T.c[0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b0, T.c[0][0], 0, 0, 0);
+        T.c[0][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b1, T.c[0][1], 0, 0, 0);
+        T.c[1][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b0, T.c[1][0], 0, 0, 0);
+        T.c[1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b1, T.c[1][1], 0, 0, 0);
     }
+    return T;
+}
+__device__ inline GjTile gj_mm(const double *A, int lda, const double *B, int ldb, double (*As)[GJB + 1],
+                               double (*Bs)[GJB + 1]) {
+    GjLoad(A, lda, B, ldb).store(As, Bs);
     __syncthreads();
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-        const int row0 = wr + lk + 4 * r, row1 = row0 + 16, col0 = wc + li, col1 = col0 + 16;
-        double *o00 = C + (size_t)row0 * ldc + col0, *o01 = C + (size_t)row0 * ldc + col1;
-        double *o10 = C + (size_t)row1 * ldc + col0, *o11 = C + (size_t)row1 * ldc + col1;
-        *o00 = acc ? *o00 + alpha * c00[r] : alpha * c00[r];
-        *o01 = acc ? *o01 + alpha * c01[r] : alpha * c01[r];
-        *o10 = acc ? *o10 + alpha * c10[r] : alpha * c10[r];
-        *o11 = acc ? *o11 + alpha * c11[r] : alpha * c11[r];
-    }
+    return gj_product(As, Bs);
 }
 
-// block row k: A_kj <- Dk A_kj (j != k)
-__global__ void __launch_bounds__(256) k_gj_row(int ld, int nb, int k, double *A, const double *Dk, double *tmp) {
+// Two pivot blocks p = 2 s, q = 2 s + 1 per pass over the matrix.  Eliminating block p with inverse Dp is
+//   A_ij -= V_i W_j,  A_pj = W_j,  A_ip = -V_i Dp,  A_pp = Dp,   W_j = Dp A_pj, V_i = A_ip (i, j != p),
+// and the same for q on the result.  Only row and column q of the first elimination are needed before the
+// second one's panels are known, so the panels of both are formed first (W, V: ld x 64 per block, kept
+// beside A) and one launch applies both to every tile.  Every entry sees the operations of two separate
+// passes in their order, so the bits are theirs, for half the traffic.
+struct GjStep {
+    int ld, nb, p;      // q = p + 1
+    double *A, *Dp, *Dq;
+    double *Wp, *Vp, *Wq, *Vq;  // W: 64 x ld (row stride ld), V: ld x 64
+    double *Rq;         // row q after the first elimination, 64 x ld
+};
+__device__ inline double *gj_tile(const GjStep &s, int i, int j) {
+    return s.A + (size_t)i * GJB * s.ld + (size_t)j * GJB;
+}
+
+// W_j = D R_j for j != k (R: a block row, row stride ld) and, for the first block, V_j = A_jk
+__global__ void __launch_bounds__(256) k_gj_panel(GjStep s, int k, const double *D, const double *R, double *W, double *V) {
     __shared__ double As[GJB][GJB + 1], Bs[GJB][GJB + 1];
     const int j = blockIdx.x;
     if (j == k) return;
-    double *Akj = A + (size_t)k * GJB * ld + (size_t)j * GJB;
-    double *T = tmp + (size_t)j * GJB * GJB;
-    tile_mm(Dk, GJB, Akj, ld, T, GJB, 1.0, false, As, Bs);
-    __syncthreads();
-    for (int e = threadIdx.x; e < GJB * GJB; e += 256) Akj[(size_t)(e / GJB) * ld + e % GJB] = T[e];
+    if (V)
+        for (int e = threadIdx.x; e < GJB * GJB; e += 256)
+            V[(size_t)j * GJB * GJB + e] = gj_tile(s, j, k)[(size_t)(e / GJB) * s.ld + e % GJB];
+    double *out = W + (size_t)j * GJB;
+    gj_mm(D, GJB, R + (size_t)j * GJB, s.ld, As, Bs).each([&](int r, int c, double v) { out[(size_t)r * s.ld + c] = v; });
 }
 
-// A_ij -= A_ik A_kj for i, j != k
-__global__ void __launch_bounds__(256) k_gj_update(int ld, int nb, int k, double *A) {
+// row and column q after the first elimination, into Rq and Vq
+__global__ void __launch_bounds__(256) k_gj_second(GjStep s) {
     __shared__ double As[GJB][GJB + 1], Bs[GJB][GJB + 1];
-    const int i = blockIdx.x / nb, j = blockIdx.x % nb;
-    if (i == k || j == k) return;
-    tile_mm(A + (size_t)i * GJB * ld + (size_t)k * GJB, ld, A + (size_t)k * GJB * ld + (size_t)j * GJB, ld,
-            A + (size_t)i * GJB * ld + (size_t)j * GJB, ld, -1.0, true, As, Bs);
+    const int q = s.p + 1, j = blockIdx.x / 2;
+    if (blockIdx.x % 2 == 0) {
+        double *out = s.Rq + (size_t)j * GJB;
+        const double *Vq = s.Vp + (size_t)q * GJB * GJB;
+        if (j == s.p) {
+            gj_mm(Vq, GJB, s.Dp, GJB, As, Bs).each([&](int r, int c, double v) { out[(size_t)r * s.ld + c] = -v; });
+        } else {
+            const double *a = gj_tile(s, q, j);
+            gj_mm(Vq, GJB, s.Wp + (size_t)j * GJB, s.ld, As, Bs).each([&](int r, int c, double v) {
+                out[(size_t)r * s.ld + c] = a[(size_t)r * s.ld + c] - v;
+            });
+        }
+    } else {
+        if (j == q) return;
+        double *out = s.Vq + (size_t)j * GJB * GJB;
+        if (j == s.p) {
+            for (int e = threadIdx.x; e < GJB * GJB; e += 256)
+                out[e] = s.Wp[(size_t)(e / GJB) * s.ld + (size_t)q * GJB + e % GJB];
+        } else {
+            const double *a = gj_tile(s, j, q);
+            gj_mm(s.Vp + (size_t)j * GJB * GJB, GJB, s.Wp + (size_t)q * GJB, s.ld, As, Bs).each([&](int r, int c, double v) {
+                out[r * GJB + c] = a[(size_t)r * s.ld + c] - v;
+            });
+        }
+    }
 }
 
-// block column k: A_ik <- -A_ik Dk (i != k), A_kk <- Dk
-__global__ void __launch_bounds__(256) k_gj_col(int ld, int nb, int k, double *A, const double *Dk, double *tmp) {
+// both eliminations on every tile.  Bound by the matrix once in and out (2 x 128 MB at nc = 3,900) and the
+// matrix pipe behind one workgroup barrier per product: 115 us per 128 pivots, 2 x 88 with one block a pass
+__global__ void __launch_bounds__(256) k_gj_update(GjStep s) {
     __shared__ double As[GJB][GJB + 1], Bs[GJB][GJB + 1];
-    const int i = blockIdx.x;
-    double *Aik = A + (size_t)i * GJB * ld + (size_t)k * GJB;
-    if (i == k) {
-        for (int e = threadIdx.x; e < GJB * GJB; e += 256) Aik[(size_t)(e / GJB) * ld + e % GJB] = Dk[e];
+    const int i = blockIdx.x / s.nb, j = blockIdx.x % s.nb, p = s.p, q = p + 1;
+    double *C = gj_tile(s, i, j);
+    const size_t vi = (size_t)i * GJB * GJB, wj = (size_t)j * GJB;
+    auto copy = [&](const double *src, int lds) {
+        for (int e = threadIdx.x; e < GJB * GJB; e += 256) C[(size_t)(e / GJB) * s.ld + e % GJB] = src[(size_t)(e / GJB) * lds + e % GJB];
+    };
+    if (i == q) {
+        if (j == q) copy(s.Dq, GJB);
+        else copy(s.Wq + wj, s.ld);
         return;
     }
-    double *T = tmp + (size_t)i * GJB * GJB;
-    tile_mm(Aik, ld, Dk, GJB, T, GJB, -1.0, false, As, Bs);
+    if (j == q) {
+        gj_mm(s.Vq + vi, GJB, s.Dq, GJB, As, Bs).each([&](int r, int c, double v) { C[(size_t)r * s.ld + c] = -v; });
+        return;
+    }
+    const double *Bp = j == p ? s.Dp : s.Wp + wj;
+    const int lb = j == p ? GJB : s.ld;
+    double old[16];
+    GjTile first = {};
+    if (i != p) {
+        GjLoad(s.Vp + vi, GJB, Bp, lb).store(As, Bs);
+        __syncthreads();
+    }
+    // the second product's operands and the tile itself arrive beside the first product
+    const GjLoad two(s.Vq + vi, GJB, s.Wq + wj, s.ld);
+    int n = 0;
+    first.each([&](int r, int c, double) { old[n++] = i == p ? Bp[(size_t)r * lb + c] : j == p ? 0.0 : C[(size_t)r * s.ld + c]; });
+    if (i != p) {
+        first = gj_product(As, Bs);
+        n = 0;
+        first.each([&](int, int, double v) { old[n++] -= v; });
+        __syncthreads();
+    }
+    two.store(As, Bs);
     __syncthreads();
-    for (int e = threadIdx.x; e < GJB * GJB; e += 256) Aik[(size_t)(e / GJB) * ld + e % GJB] = T[e];
+    n = 0;
+    gj_product(As, Bs).each([&](int r, int c, double v) { C[(size_t)r * s.ld + c] = old[n++] - v; });
 }
 
 // ------------------------------------------------------------------------
@@ -960,7 +1111,7 @@ static int build_two_level(Ctx &c, const double *K64, int agg, TwoLevel &t, std:
     make_aggregates(m, D, agg, nz, node_agg, na);
     t.na = na;
     t.nc = na * NM;
-    t.ld = (t.nc + GJB - 1) / GJB * GJB;
+    t.ld = (t.nc + GJP - 1) / GJP * GJP;
     // aggregate -> nodes, centroids, mode values (scaled by the cell size)
     std::vector<int> agg_off(na + 1, 0), agg_node(nn);
     for (int a = 0; a < nn; a++) agg_off[node_agg[a] + 1]++;
@@ -1036,23 +1187,39 @@ static int build_two_level(Ctx &c, const double *K64, int agg, TwoLevel &t, std:
                            c.stream));
     PDX_HIP(hipMemcpyAsync(t.Pn, Pn.data(), Pn.size() * 8, hipMemcpyHostToDevice, c.stream));
     PDX_HIP(hipMemcpyAsync(blk_slot_d, blk_slot.data(), blk_slot.size() * 4, hipMemcpyHostToDevice, c.stream));
-    k_coarse_ap<D, NM><<<(nn + 127) / 128, 128, 0, c.stream>>>(nn, c.adj_off, c.adj, K64, t.Pn, blk_slot_d, t.kp_off,
+    k_coarse_ap<D, NM><<<(nn + AP_NODES<D, NM> - 1) / AP_NODES<D, NM>, 256, 0, c.stream>>>(nn, c.adj_off, c.adj, K64, t.Pn, blk_slot_d, t.kp_off,
                                                                 c.eq, t.kp);
     // dense Galerkin matrix; padding rows/columns stay zero and drop out of the inverse
-    double *A = t.Ainv, *diag0, *Dk, *tmpb;
-    if ((rc = tl_alloc(t, diag0, t.ld, err)) || (rc = tl_alloc(t, Dk, GJB * GJB, err)) ||
-        (rc = tl_alloc(t, tmpb, (size_t)t.ld * GJB, err)))
-        return rc;
+    double *A = t.Ainv, *diag0, *work;
+    const size_t panel = (size_t)t.ld * GJB;
+    if ((rc = tl_alloc(t, diag0, t.ld, err)) || (rc = tl_alloc(t, work, 5 * panel + 2 * GJB * GJB, err))) return rc;
     k_fill_d<<<2048, 256, 0, c.stream>>>((size_t)t.ld * t.ld, A, 0.0);
-    k_coarse_galerkin<D, NM><<<(t.nc + 63) / 64, 64, 0, c.stream>>>(na, t.agg_off, t.agg_node, t.Pn, t.kp_off,
-                                                                    t.kp_agg, t.kp, t.ld, A);
+    const size_t bits = (size_t)(na + 31) / 32 * sizeof(unsigned);
+    if (bits > 128 * 1024) { err = "too many aggregates for the coarse space"; return PDX_ERR_LIMIT; }
+    PDX_HIP(hipFuncSetAttribute((const void *)k_coarse_galerkin<D, NM>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bits));
+    k_coarse_galerkin<D, NM><<<na, 1024, bits, c.stream>>>(na, t.agg_off, t.agg_node, t.Pn, t.kp_off, t.kp_agg, t.kp, t.ld, A);
     k_diag_copy<<<(t.ld + 255) / 256, 256, 0, c.stream>>>(t.ld, t.ld, A, diag0);
     const int nb = t.ld / GJB;
-    for (int k = 0; k < nb; k++) {
-        k_gj_diag<<<1, 1024, 0, c.stream>>>(t.ld, k, A, diag0, Dk);
-        k_gj_row<<<nb, 256, 0, c.stream>>>(t.ld, nb, k, A, Dk, tmpb);
-        k_gj_update<<<nb * nb, 256, 0, c.stream>>>(t.ld, nb, k, A);
-        k_gj_col<<<nb, 256, 0, c.stream>>>(t.ld, nb, k, A, Dk, tmpb);
+    GjStep g;
+    g.ld = t.ld;
+    g.nb = nb;
+    g.A = A;
+    g.Wp = work;
+    g.Vp = work + panel;
+    g.Wq = work + 2 * panel;
+    g.Vq = work + 3 * panel;
+    g.Rq = work + 4 * panel;
+    g.Dp = work + 5 * panel;
+    g.Dq = g.Dp + GJB * GJB;
+    for (g.p = 0; g.p < nb; g.p += 2) {
+        const int q = g.p + 1;
+        const double *row = A + (size_t)g.p * GJB * t.ld;
+        k_gj_diag<<<1, 256, 0, c.stream>>>(row + (size_t)g.p * GJB, t.ld, diag0 + (size_t)g.p * GJB, g.Dp);
+        k_gj_panel<<<nb, 256, 0, c.stream>>>(g, g.p, g.Dp, row, g.Wp, g.Vp);
+        k_gj_second<<<2 * nb, 256, 0, c.stream>>>(g);
+        k_gj_diag<<<1, 256, 0, c.stream>>>(g.Rq + (size_t)q * GJB, t.ld, diag0 + (size_t)q * GJB, g.Dq);
+        k_gj_panel<<<nb, 256, 0, c.stream>>>(g, q, g.Dq, g.Rq, g.Wq, nullptr);
+        k_gj_update<<<nb * nb, 256, 0, c.stream>>>(g);
     }
     PDX_HIP(hipGetLastError());
     PDX_HIP(hipStreamSynchronize(c.stream));
