@@ -468,6 +468,7 @@ void ctx_free(Ctx *c) {
     if (c->K32) hipFree(c->K32);
     if (c->nlm_F) hipFree(c->nlm_F);
     if (c->nlm_a) hipFree(c->nlm_a);
+    if (c->nlm_M) hipFree(c->nlm_M);
     if (c->dofs_tmp) hipFree(c->dofs_tmp);
     if (c->K32s) hipFree(c->K32s);
     if (c->K64s) hipFree(c->K64s);

@@ -163,6 +163,7 @@ struct Ctx {
     // consistent-mass explicit steps (LUMPMASS OFF): F = F_ext - K u_n and the acceleration of
     // M a = F, full DOF vectors; the acceleration warm-starts the next step's solve
     double *nlm_F = nullptr, *nlm_a = nullptr;
+    double *nlm_M = nullptr;  // [nblk] the mass of a node pair: M's blocks are scalar multiples of I
     long long nlm_iters = 0;  // CG iterations of the mass solves so far
     double *dofs_tmp = nullptr;  // [nn*d] DOF values of the last stored step (stress input)
 
@@ -239,6 +240,8 @@ struct Mirrored {
     // the operator is ks K + ms M (M: the consistent mass) of this context, so that its products may be
     // formed from the elements and families (hex.hpp); ks = 0: some other matrix
     double ks = 0.0, ms = 0.0;
+    // FP64 operator whose blocks are mass[b] I: its products read these instead of the blocks
+    const double *mass = nullptr;
 };
 // exact: every mirrored lower block of A (dd*nblk values, K's block order) equals its partner's
 // transpose bit for bit (checked on the device; synchronises the stream)

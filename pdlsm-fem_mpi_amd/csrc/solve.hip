@@ -571,7 +571,9 @@ static int explicit_step_nlm(Ctx &c, int prec, int startup, std::string &err) {
     o.max_iter = 5000;
     o.warm_start = 1;
     pdx_solve_stats st{};
-    int rc = dev_solve_mat(c, c.Mk, nullptr, o, c.nlm_F, c.nlm_a, st, err);
+    Mirrored mir;
+    mir.mass = c.nlm_M;
+    int rc = dev_solve_mat(c, c.Mk, nullptr, o, c.nlm_F, c.nlm_a, st, err, &mir);
     c.nlm_iters += st.iterations;
     if (rc) return rc;
     const int n = c.nn * c.dim;
@@ -581,6 +583,11 @@ static int explicit_step_nlm(Ctx &c, int prec, int startup, std::string &err) {
     c.step_phase = (p + 1) % 3;
     c.steps_done = s;
     return PDX_OK;
+}
+
+__global__ void k_block_scalar(size_t nblk, int dd, const double *M, double *m) {
+    for (size_t b = blockIdx.x * (size_t)blockDim.x + threadIdx.x; b < nblk; b += (size_t)gridDim.x * blockDim.x)
+        m[b] = M[b * dd];
 }
 
 // K (and the FP32 / row-local / mirrored copies the step reads) for the current bond states;
@@ -609,9 +616,15 @@ static int explicit_operators(Ctx &c, int prec, bool lumped, std::string &err) {
         if (e) return e;
     }
     if (!lumped) {
-        if (!c.Mk_valid) {
+        const bool fresh = !c.Mk_valid;
+        if (fresh) {
             int e = dev_mass_on_K(c, err);
             if (e) return e;
+        }
+        if (fresh || !c.nlm_M) {
+            if (!c.nlm_M) PDX_HIP(hipMalloc((void **)&c.nlm_M, sizeof(double) * std::max<long long>(c.nblk, 1)));
+            k_block_scalar<<<2048, 256, 0, c.stream>>>((size_t)c.nblk, c.dd, c.Mk, c.nlm_M);
+            PDX_HIP(hipGetLastError());
         }
         const size_t n = (size_t)c.nn * c.dim;
         if (!c.nlm_F) {
