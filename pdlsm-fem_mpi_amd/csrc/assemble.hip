@@ -1117,18 +1117,13 @@ static int family_args(Ctx &c, int *status, FamArgs &A, size_t &lds, std::string
     return PDX_OK;
 }
 
-// Bond weights and inverse shape tensors for the products by moments, for the bond states K was
-// assembled with
+// Bond weights and inverse shape tensors for the products by moments (arrays of the tiles, hex.hip), for
+// the bond states K was assembled with
 int dev_family_moments(Ctx &c, std::string &err) {
     if (c.mom_gen == c.K_gen) return PDX_OK;
     FamArgs A;
     size_t lds = 0;
     if (int rc = family_args(c, c.asm_status, A, lds, err)) return rc;
-    if (!c.mom_w) {
-        const size_t nmem = c.host->fam_mem.size();
-        PDX_HIP(hipMalloc((void **)&c.mom_w, std::max<size_t>(nmem, 1) * sizeof(double)));
-        PDX_HIP(hipMalloc((void **)&c.mom_T, std::max<size_t>((size_t)c.nfam * 54, 1) * sizeof(double)));
-    }
     A.fam_w = c.mom_w;
     A.fam_T = c.mom_T;
     PDX_HIP(hipFuncSetAttribute((const void *)k_family<3, true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));

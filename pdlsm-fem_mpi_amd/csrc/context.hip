@@ -339,10 +339,6 @@ int ctx_build(const Model &m, int device, Ctx *&out, std::string &err) {
                 if (!((pd_bits[(size_t)q >> 3] >> (q & 7)) & 1) && fcnt[q + 1] == fcnt[q]) bare++;
             c->k_needs_fill = bare > 0;
         }
-        if (D == 3) {
-            c->nfe_off_host = std::move(cnt);
-            c->nfe_item_host = std::move(item);
-        }
         // all elements (lumped mass)
         std::vector<int> acnt(m.nn + 1, 0);
         for (int e = 0; e < m.ne; e++)
@@ -480,8 +476,6 @@ void ctx_free(Ctx *c) {
     if (c->learned_Minv) hipFree(c->learned_Minv);
     if (c->gnn_keff) hipFree(c->gnn_keff);
     if (c->fam_c) hipFree(c->fam_c);
-    if (c->mom_w) hipFree(c->mom_w);
-    if (c->mom_T) hipFree(c->mom_T);
     if (c->Kown32) hipFree(c->Kown32);
     if (c->Kown64) hipFree(c->Kown64);
     if (c->stress_stage) hipFree(c->stress_stage);

@@ -170,9 +170,9 @@ struct Ctx {
     // node tiles of the products with hex8 elements without their K blocks (hex.hip)
     void *hex = nullptr;
     bool hex_tried = false;
-    std::vector<int> nfe_off_host, nfe_item_host;  // nfe_off, nfe_item (3D), until the tiles are built
     // PD rows formed from the moments of their families (hex.hpp): bond weights [members] and the
-    // second-order rows of the inverse shape tensors [nfam * 54], for the K of generation mom_gen
+    // second-order rows of the inverse shape tensors [nfam * 54], for the K of generation mom_gen;
+    // allocated and freed with the tiles
     double *mom_w = nullptr, *mom_T = nullptr;
     long long mom_gen = -1;
     int tune_seen[2] = {-1, -1};  // form the tuner found for a context that steps through the tiles

@@ -6,6 +6,7 @@
 #include <bitset>
 #include <cmath>
 #include <cstring>
+#include <new>
 #include <numeric>
 #include <vector>
 
@@ -286,35 +287,61 @@ void hex_tiles_host(const Model &m, const std::vector<int> &nfe_off, const std::
         for (size_t q = 0; q < list[x].size(); q++) H.work[q * 8 + x] = list[x][q];
 }
 
-int hex_tiles(Ctx &c, const HexTiles *&out, std::string &err) {
-    out = (const HexTiles *)c.hex;
-    if (c.hex_tried) return PDX_OK;
-    HexTilesHost H;
-    if (c.dim == 3 && c.host && c.host->dim == 3) hex_tiles_host(*c.host, c.nfe_off_host, c.nfe_item_host, HEX_MIN_NODES, H);
-    c.nfe_off_host = std::vector<int>();
-    c.nfe_item_host = std::vector<int>();
-    if (H.tile.empty()) {
-        c.hex_tried = true;
-        return PDX_OK;
-    }
+// The device arrays of the tiles, and those of the family moments, which only products through the
+// tiles read.  The incidence lists come back from the device (7 MB of a 60^3 box), so no copy of them
+// waits on the host.
+static int build_hex_tiles(Ctx &c, HexTilesHost &H, std::string &err) {
+    std::vector<int> off((size_t)c.nn + 1), item;
+    PDX_HIP(hipMemcpy(off.data(), c.nfe_off, off.size() * sizeof(int), hipMemcpyDeviceToHost));
+    item.resize((size_t)off[c.nn]);
+    if (!item.empty()) PDX_HIP(hipMemcpy(item.data(), c.nfe_item, item.size() * sizeof(int), hipMemcpyDeviceToHost));
+    hex_tiles_host(*c.host, off, item, HEX_MIN_NODES, H);
+    if (H.tile.empty()) return PDX_OK;
     auto *T = new HexTiles();
     c.hex = T;
     T->n_work = (int)H.work.size();
     T->n_fam = (int)H.fams.size();
+    auto alloc = [&](auto *&dst, size_t n) -> int {
+        const hipError_t e = hipMalloc((void **)&dst, std::max<size_t>(n, 1) * sizeof(*dst));
+        if (e == hipSuccess) return PDX_OK;
+        dst = nullptr;
+        (void)hipGetLastError();
+        err = std::string("element tiles: ") + hipGetErrorString(e);
+        return e == hipErrorOutOfMemory ? PDX_ERR_LIMIT : PDX_ERR_HIP;
+    };
     auto up = [&](auto *&dst, const auto &src) -> int {
-        PDX_HIP(hipMalloc((void **)&dst, std::max<size_t>(src.size(), 1) * sizeof(src[0])));
+        if (int rc = alloc(dst, src.size())) return rc;
         if (!src.empty()) PDX_HIP(hipMemcpy(dst, src.data(), src.size() * sizeof(src[0]), hipMemcpyHostToDevice));
         return PDX_OK;
     };
     int rc;
-    if ((rc = up(T->nodes, H.nodes)) || (rc = up(T->conn, H.conn)) ||
-        (rc = up(T->rows, H.rows)) ||
-        (rc = up(T->work, H.work)) || (rc = up(T->fams, H.fams))) {
-        free_hex_tiles(c);
+    if ((rc = up(T->nodes, H.nodes)) || (rc = up(T->conn, H.conn)) || (rc = up(T->rows, H.rows)) ||
+        (rc = up(T->work, H.work)) || (rc = up(T->fams, H.fams)))
         return rc;
+    if (T->n_fam && ((rc = alloc(c.mom_w, c.host->fam_mem.size())) || (rc = alloc(c.mom_T, (size_t)c.nfam * 54)))) return rc;
+    return PDX_OK;
+}
+
+int hex_tiles(Ctx &c, const HexTiles *&out, std::string &err) {
+    out = (const HexTiles *)c.hex;
+    if (c.hex_tried) return PDX_OK;
+    if (c.dim == 3 && c.nn >= HEX_MIN_NODES && c.host && c.host->dim == 3) {
+        HexTilesHost H;
+        int rc;
+        try {
+            rc = build_hex_tiles(c, H, err);
+        } catch (const std::bad_alloc &) {
+            rc = PDX_ERR_LIMIT;
+        }
+        if (rc) {
+            free_hex_tiles(c);
+            // out of memory: the walk of K needs none of these arrays, so this context keeps to it
+            if (rc != PDX_ERR_LIMIT) return rc;
+            err.clear();
+        }
     }
     c.hex_tried = true;
-    out = T;
+    out = (const HexTiles *)c.hex;
     return PDX_OK;
 }
 
@@ -323,6 +350,11 @@ void free_hex_tiles(Ctx &c) {
     if (!T) return;
     for (void *p : {(void *)T->nodes, (void *)T->conn, (void *)T->rows, (void *)T->work, (void *)T->fams})
         if (p) hipFree(p);
+    for (double **p : {&c.mom_w, &c.mom_T}) {
+        if (*p) hipFree(*p);
+        *p = nullptr;
+    }
+    c.mom_gen = -1;
     delete T;
     c.hex = nullptr;
     c.hex_tried = false;
