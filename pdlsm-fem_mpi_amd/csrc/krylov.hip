@@ -787,7 +787,7 @@ __global__ void __launch_bounds__(1024) k_coarse_galerkin(int na, const int *agg
                                                           const double *kp, int ld, double *Ac) {
     extern __shared__ unsigned gbits[];  // [(na + 31) / 32]
     constexpr int JM = 512, NC = 256, LJ = 8;
-    __shared__ int jl[JM], njs, node[NC], first[NC], count[NC], lj[NC][LJ];
+    __shared__ int jl[JM], njs, word, node[NC], first[NC], count[NC], lj[NC][LJ];
     const int I = blockIdx.x, t = threadIdx.x, words = (na + 31) / 32;
     const int n0 = agg_off[I], n1 = agg_off[I + 1];
     for (int w = t; w < words; w += blockDim.x) gbits[w] = 0;
@@ -799,18 +799,18 @@ __global__ void __launch_bounds__(1024) k_coarse_galerkin(int na, const int *agg
             atomicOr(&gbits[J >> 5], 1u << (J & 31));
         }
     }
-    for (int done = 0;;) {  // JM aggregates at a time
+    for (int done = 0;;) {  // JM aggregates at a time, from word `done` of the bits
         __syncthreads();
         if (t == 0) {
             int n = 0;
             for (int w = done; w < words && n + 32 <= JM; done = ++w)
                 for (unsigned v = gbits[w]; v; v &= v - 1) jl[n++] = w * 32 + __ffs(v) - 1;
             njs = n;
-            jl[JM - 1] = done;  // the list is never that long: the next word to look at
+            word = done;
         }
         __syncthreads();
         const int nj = njs;
-        done = jl[JM - 1];
+        done = word;
         for (int v0 = 0; v0 < nj * NM * NM; v0 += blockDim.x) {
             const int v = v0 + t, e = v % (NM * NM), m = e / NM, m2 = e % NM;
             const int J = v < nj * NM * NM ? jl[v / (NM * NM)] : -1;

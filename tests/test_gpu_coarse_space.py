@@ -27,3 +27,23 @@ def test_coarse_correction_is_exact_on_translations(dim, agg):
     total, scale = np.abs(y.sum(1)), np.abs(y).sum(1)
     print(f"dim {dim} agg {agg}: {(total / scale).max():.1e}", flush=True)
     assert (total <= 2.0 ** -23 * scale).all(), (total / scale).max()
+
+
+@pytest.mark.parametrize("n", [8, 9])
+def test_aggregates_that_reach_512_others(n):
+    """A PD body inside every node's horizon with one node per aggregate: each row of the Galerkin matrix holds all
+    512 (one full list of the kernel) or 729 (two lists) aggregates.  The coarse space is then the whole space, so
+    Q is K's inverse and y = K (I - Q K) z is rounding: with a condition number below 1e7 (1.0e6 for 729 nodes,
+    asserted on the host), under 1e7 * 1e-16 * some 1e3 operations = 1e-6 of K's entries.  A lost 3 x 3 block
+    column leaves 0.1."""
+    import scipy.sparse as sp
+    model = pdx.Model(W.box3d(n=n, pd_block=n, jitter=0.0, m=30.0))
+    assert model.max_family == n ** 3
+    cx = pdx.Context(model)
+    ia, ja = model.csr()
+    K = sp.csr_matrix((cx.assemble(pdx.PDX_MODE_STATIC)[0], ja, ia), shape=(model.neq, model.neq)).toarray()
+    assert np.linalg.cond(K) < 1e7
+    y = pdx.gnn_inputs(cx, n_probes=2, probe_seed=n, coarse_agg=1)["y"].astype(np.float64)
+    ratio = np.abs(y).max() / np.abs(K).max()
+    print(f"n {n}: {ratio:.1e}", flush=True)
+    assert ratio <= 1e-6
