@@ -237,8 +237,9 @@ int dev_spmv_K(Ctx &c, const double *K64, const double *x, double *y);
 struct Mirrored {
     const double *K64 = nullptr;
     const float *K32 = nullptr;
-    // the operator is ks K + ms M (M: the consistent mass) of this context, so that its products may be
-    // formed from the elements and families (hex.hpp); ks = 0: some other matrix
+    // context_op: the operator is ks K + ms M (M: the consistent mass) of this context, so that its
+    // products may be formed from the elements and families (hex.hpp); ks may be 0 (Newmark with beta = 0)
+    bool context_op = false;
     double ks = 0.0, ms = 0.0;
     // FP64 operator whose blocks are mass[b] I: its products read these instead of the blocks
     const double *mass = nullptr;

@@ -1890,7 +1890,7 @@ static int solve_masked(Ctx &c, const double *K64, const float *K32, const pdx_s
     op64.src = src64;
     op32.src = src32;
     op64.mass = mir.mass;
-    if (D == 3 && mir.ks != 0.0) {
+    if (D == 3 && mir.context_op) {
         if (int rc = product_tiles(c, o.precision, op64.ht, err)) return rc;
         op64.A64 = K64;
         op64.ks = mir.ks;
@@ -2091,6 +2091,7 @@ int dev_solve(Ctx &c, const pdx_solve_opts &o, const double *b_dev, double *x_de
     Mirrored mir;
     // mirrored storage is for products that walk the blocks
     if (o.mirrored && c.dim > 1 && !tiles && (rc = kown_for_solve(c, o.precision, mir, err))) return rc;
+    mir.context_op = true;
     mir.ks = 1.0;
     return dev_solve_mat(c, c.K, walk32 ? c.K32 : nullptr, o, b_dev, x_dev, st, err, &mir);
 }

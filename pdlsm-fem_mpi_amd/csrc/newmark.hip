@@ -298,6 +298,7 @@ int dev_newmark(Ctx &c, int nsteps, const pdx_solve_opts &o, std::vector<double>
     // mirrored storage of K_eff for the SpMVs, when its mirrored blocks are exact transposes
     // (K's are by construction; the consistent mass's are checked with them)
     Mirrored mir;
+    mir.context_op = true;
     mir.ks = c.beta * c.dt * c.dt;
     mir.ms = 1.0;
     double *own64 = nullptr;

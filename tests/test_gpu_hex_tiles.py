@@ -142,3 +142,22 @@ def test_fp32_newmark_through_tiles():
     assert run[1][3]["converged"] and run[1][3]["refinements"] > 0
     for x, y in zip(run[0][:3], run[1][:3]):
         assert rel(y, x) <= 1e-8
+
+
+@pytest.mark.parametrize("n, precision", [(65, pdx.PDX_FP32), (29, pdx.PDX_FP64)])
+def test_newmark_with_beta_zero(n, precision):
+    """beta = 0: the operator of a step is M alone (no K in it), above the sizes where its products go through the tiles.
+    The acceleration solves M a = F to the tolerance asked for, checked with the assembled M."""
+    mesh = _dt(W.box3d(n=n, pd_block=8))
+    mesh["beta"] = 0.0
+    mesh["nbc"][0]["val"] = 1e6
+    model = pdx.Model(mesh)
+    cx = pdx.Context(model)
+    _, _, a, st = cx.newmark_run(1, pdx.solve_opts(precond=pdx.PDX_PREC_BLOCK_JACOBI, precision=precision, tol=1e-8))
+    assert st["converged"]
+    M = _csr(model, cx.mass_on_K())
+    dU = model.values()
+    for s in mesh["ebc"]:
+        dU[(np.asarray(s["nid"]) - 1) * 3 + s["dof"]] += mesh["dt"] * s.get("vel", 0.0) * bool(s.get("vary", False))
+    F = pdx.Context(model).assemble(pdx.PDX_MODE_NEWMARK, UN=dU)[1]
+    assert np.linalg.norm(F - M @ a) <= (1e-8 + 1e-11) * np.linalg.norm(F)
