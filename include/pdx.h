@@ -423,6 +423,11 @@ int pdx_explicit_tuning(pdx_ctx *c, int precision, int *lanes, int *nontemporal,
  * choice (or the products without K), or -1 to choose again at the next step; forms with the same lanes per row compute the
  * same bits, the lanes per row change the order of the row sum */
 int pdx_explicit_set_form(pdx_ctx *c, int precision, int form);
+/* the products of a large 3D model formed without most of K, so far: counts[0] node tiles, [1] hex8
+ * elements they compute (one between two tiles counts in both), [2] families formed from their moments,
+ * [3] rows walked in K beside them, [4] products launched (one captured in a graph counts once).  All 0
+ * while every product walks K.  Reads counters only: nothing is built */
+int pdx_tile_counts(const pdx_ctx *c, long long counts[5]);
 
 #ifdef __cplusplus
 }

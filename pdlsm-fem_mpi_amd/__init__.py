@@ -113,6 +113,7 @@ EXPORTS = {
     "pdx_last_timing": (_I, [_P, _P, _P]),
     "pdx_explicit_tuning": (_I, [_P, _I, _P, _P, _P, _P, _P, _P, _P, _P, _P]),
     "pdx_explicit_set_form": (_I, [_P, _I, _I]),
+    "pdx_tile_counts": (_I, [_P, _P]),
     "pdx_node_stresses": (_I, [_P, _P, _P]),
     "pdx_node_stresses_timed": (_I, [_P, _P, _P]),
     "pdx_node_stresses_noalloc": (_I, [_P, _P, _P]),
@@ -466,6 +467,13 @@ class Context:
                                        C.byref(rel), C.byref(sym), C.byref(alt), C.byref(form), _p(ms)))
         return (lanes.value, bool(nt.value), bool(xm.value), bool(soa.value), bool(rel.value), bool(sym.value),
                 ms, bool(alt.value), form.value)
+
+    def tile_counts(self):
+        """Products formed without most of K so far (large 3D models): node tiles, elements they compute, families
+        formed from their moments, rows walked in K beside them, products launched; all 0 while every product walks K."""
+        n = np.zeros(5, np.int64)
+        _chk(lib().pdx_tile_counts(self.h, _p(n)))
+        return dict(zip(("tiles", "elements", "families", "rows", "products"), n.tolist()))
 
     def max_eig(self, iters=100):
         v = C.c_double(0)

@@ -11,6 +11,7 @@
 
 #include "../../include/pdx.h"
 #include "device.hpp"
+#include "hex.hpp"
 #include "setup.hpp"
 
 namespace pdx {
@@ -24,7 +25,6 @@ int dev_newmark(Ctx &c, int nsteps, const pdx_solve_opts &o, std::vector<double>
 int dev_explicit_state(Ctx &c, double *u_out, double *u_prev, std::string &err);
 int dev_max_eig(Ctx &c, int iters, double *lmax, std::string &err);
 int explicit_tune_seen(Ctx &c, int pi, std::string &err);
-void free_hex_tiles(Ctx &c);
 int stress_scratch_init(int device, std::string &err);
 int dev_node_stresses_noalloc(Ctx &c, const double *u_dev, double *sigma_dev, std::string &err);
 
@@ -992,6 +992,14 @@ int pdx_explicit_set_form(pdx_ctx *pc, int precision, int form) {
         hipGraphExecDestroy(c.graph[precision]);
         c.graph[precision] = nullptr;
     }
+    return PDX_OK;
+}
+
+int pdx_tile_counts(const pdx_ctx *pc, long long *counts) {
+    if (!pc || !counts) return fail(PDX_ERR_ARG, "null argument");
+    const auto *t = (const HexTiles *)pc->c->hex;
+    const long long v[5] = {t ? t->n_tile : 0, t ? t->n_ele : 0, t ? t->n_fam : 0, t ? t->n_row : 0, pc->c->hex_products};
+    std::copy(v, v + 5, counts);
     return PDX_OK;
 }
 

@@ -170,6 +170,7 @@ struct Ctx {
     // node tiles of the products with hex8 elements without their K blocks (hex.hip)
     void *hex = nullptr;
     bool hex_tried = false;
+    long long hex_products = 0;  // launched or captured so far
     // PD rows formed from the moments of their families (hex.hpp): bond weights [members] and the
     // second-order rows of the inverse shape tensors [nfam * 54], for the K of generation mom_gen;
     // allocated and freed with the tiles

@@ -236,6 +236,7 @@ void hex_tiles_host(const Model &m, const std::vector<int> &nfe_off, const std::
         for (int c = 0; c < 3; c++) h.x[c] = m.x[(size_t)all[k]->node[0] * 3 + c];
         n_node += all[k]->node.size();
         n_ele += all[k]->place.size();
+        H.n_ele += (long long)all[k]->ele.size();
         H.tile[k] = h;
     }
     H.nodes.resize(n_node);
@@ -301,6 +302,9 @@ static int build_hex_tiles(Ctx &c, HexTilesHost &H, std::string &err) {
     c.hex = T;
     T->n_work = (int)H.work.size();
     T->n_fam = (int)H.fams.size();
+    T->n_tile = (int)H.tile.size();
+    T->n_row = (int)H.rows.size();
+    T->n_ele = H.n_ele;
     auto alloc = [&](auto *&dst, size_t n) -> int {
         const hipError_t e = hipMalloc((void **)&dst, std::max<size_t>(n, 1) * sizeof(*dst));
         if (e == hipSuccess) return PDX_OK;

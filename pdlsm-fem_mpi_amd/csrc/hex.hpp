@@ -39,6 +39,8 @@ struct HexTiles {
     int *rows = nullptr;  // rows formed from K, a wavefront each
     int n_fam = 0;
     int *fams = nullptr;  // families whose rows hold nothing but their bonds, 16 lanes each
+    int n_tile = 0, n_row = 0;
+    long long n_ele = 0;  // elements of all tiles
 };
 constexpr int HEX_ROWS = HT_THREADS / 64;  // rows of a block
 constexpr int HEX_FAMS = HT_THREADS / 16;  // families of a block
@@ -47,6 +49,7 @@ struct HexTilesHost {
     std::vector<HexTile> tile, work;
     std::vector<int> nodes, rows, fams;
     std::vector<unsigned short> conn;
+    long long n_ele = 0;
 };
 void hex_tiles_host(const Model &m, const std::vector<int> &nfe_off, const std::vector<int> &nfe_item, long long min_nodes,
                     HexTilesHost &H);

@@ -1544,6 +1544,7 @@ template <typename V>
 static void launch_spmv_hex(Ctx &c, const Product &P, const V *x, V *y, const V *w0, double *bp0, const V *w1,
                             double *bp1) {
     const double lam8 = P.ks * c.lambda / 8, mu8 = P.ks * c.mu / 8, rho8 = P.ms * c.rho / 8;
+    c.hex_products++;
 #define PDX_SPMV_HEX(MASS)                                                                                        \
     k_spmv_hex<V, MASS><<<P.ht->n_work, HT_THREADS, 0, c.stream>>>(                                               \
         *P.ht, moment_args(c), P.ks, lam8, mu8, rho8, P.ms * c.rho, c.adj_off, c.adj, P.A64, c.x, x, y, c.eq, w0, bp0, w1, \

@@ -466,6 +466,7 @@ static int step_tiles(Ctx &c, int pi, const HexTiles *&ht, std::string &err) {
 template <bool FO>
 static void launch_explicit_hex(Ctx &c, const HexTiles &ht, const double *Un, const double *Unm1, double *Unp1,
                                 const double *nbc_cur, double *nbc_next, int startup) {
+    c.hex_products++;
     k_explicit_hex<FO><<<ht.n_work, HT_THREADS, 0, c.stream>>>(
         ht, moment_args(c), c.lambda / 8, c.mu / 8, c.adj_off, c.adj, c.K, c.x, Un, Unm1, Unp1, c.mlump, c.f_unit, c.n_nbc, c.nn,
         nbc_cur, nbc_next, c.d_nbc_vel, c.eq, c.presc_set, c.d_ebc_vel, c.dt, startup);

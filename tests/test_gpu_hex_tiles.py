@@ -15,6 +15,7 @@ pdx, W = load_pdx(), workloads()
 
 
 def _dt(mesh):
+    mesh["lumped_mass"] = True  # the consistent-mass step walks K
     mesh["dt"] = 2e-8  # 1 mm elements of steel-like stiffness: a fraction of the critical step
     mesh["nbc"][0].update(vel=1e12, vary=True)
     mesh["ebc"][0].update(vel=1e-3, vary=True)
@@ -65,6 +66,15 @@ CASES = {
 }
 
 
+def _tiled(cx, model, name=""):
+    """The products went through the tiles, which hold every row that they may."""
+    n = cx.tile_counts()
+    assert n["products"] > 0 and n["tiles"] > 0 and n["elements"] >= (model.nfe if name != "with_tets" else 1)
+    assert (n["families"] > 0) == (model.nfam > 0)
+    if not model.npde:
+        assert n["rows"] == 0
+
+
 @pytest.mark.parametrize("name", list(CASES))
 def test_explicit_through_tiles_equals_walk_of_K(name):
     model = pdx.Model(_dt(CASES[name]()))
@@ -83,6 +93,8 @@ def test_explicit_through_tiles_equals_walk_of_K(name):
     assert rel(tiles.explicit_run(6)[0], walk.explicit_run(6)[0]) <= 1e-12
     tiles.explicit_set_form(pdx.PDX_FP64, -1)
     assert rel(tiles.explicit_run(6)[0], walk.explicit_run(6)[0]) <= 1e-12
+    _tiled(tiles, model, name)
+    assert walk.tile_counts()["products"] == 0
     assert 0 <= tiles.explicit_tuning_full(pdx.PDX_FP64)[8] < pdx.EXPLICIT_FORMS
     assert rel(tiles.explicit_run(6)[0], walk.explicit_run(6)[0]) <= 1e-12
 
@@ -97,6 +109,8 @@ def test_fp32_force_through_tiles():
     e_tiles = rel(tiles.explicit_run(25, pdx.PDX_FP32)[0], u)
     e_walk = rel(walk.explicit_run(25, pdx.PDX_FP32)[0], u)
     assert e_tiles <= 1.2 * e_walk <= 1e-6
+    _tiled(tiles, model)
+    assert ref.tile_counts()["products"] == walk.tile_counts()["products"] == 0
 
 
 def _csr(model, values):
@@ -130,16 +144,63 @@ def test_solves_through_tiles(name, opts):
     assert np.linalg.norm(F - keff @ a) <= (1e-8 + 1e-11) * np.linalg.norm(F)
     assert st["converged"]
     u, st = fresh.static_solve(pdx.solve_opts(**o))
+    if o.get("precision") == pdx.PDX_FP32:  # at these sizes FP32 products walk the blocks
+        assert cx.tile_counts()["products"] == fresh.tile_counts()["products"] == 0
+    else:
+        _tiled(cx, model, name)
+        _tiled(fresh, model, name)
     b = fresh.assemble(pdx.PDX_MODE_STATIC)[1]
     assert np.linalg.norm(b - K @ u) <= (1e-8 + 1e-11) * np.linalg.norm(b)
+
+
+def test_fp32_two_level_through_tiles():
+    """A static solve with FP32 vectors and the two-level preconditioner at a size where FP32 products go through the
+    tiles; the residual is formed by another context's walk of K."""
+    mesh = W.box3d(n=65, pd_block=12)
+    model = pdx.Model(mesh)
+    cx = pdx.Context(model)
+    u, st = cx.static_solve(pdx.solve_opts(precision=pdx.PDX_FP32, precond=pdx.PDX_PREC_TWO_LEVEL, tol=1e-8))
+    assert st["converged"] and st["refinements"] > 0
+    _tiled(cx, model)
+    walk = pdx.Context(model)
+    b = walk.assemble(pdx.PDX_MODE_STATIC, want_K=False)[1]
+    full, eq = model.values(), model.nodes()["eq"].ravel()
+    full[eq >= 0] = u[eq[eq >= 0]]
+    walk.set_dof_values(full)
+    r = walk.assemble(pdx.PDX_MODE_EXPLICIT)[1]  # F_ext - K u
+    assert walk.tile_counts()["products"] == 0
+    assert np.linalg.norm(r) <= (1e-8 + 1e-11) * np.linalg.norm(b)
+
+
+def test_several_natural_bc_sets_through_tiles():
+    """Three traction sets (constant, ramped, on two faces) and a ramped prescribed face."""
+    mesh = _dt(W.box3d(n=30, pd_block=8))
+    n = 30
+    nid = lambda i, j, k: i + n * (j + n * k) + 1
+    side = [[nid(n - 1, j, k), nid(n - 1, j + 1, k), nid(n - 1, j + 1, k + 1), nid(n - 1, j, k + 1)]
+            for j in range(n - 1) for k in range(n - 1)]
+    top = np.asarray(mesh["nbc"][0]["con"])
+    mesh["nbc"] = [dict(con=top[::2], val=3e5, vel=0.0, vary=False), dict(con=top, val=0.0, vel=2e12, vary=True),
+                   dict(con=np.asarray(side, np.int32), val=-1e5, vel=1e12, vary=True)]
+    model = pdx.Model(mesh)
+    tiles, walk = pdx.Context(model), pdx.Context(model)
+    walk.explicit_set_form(pdx.PDX_FP64, 0)
+    for steps in (1, 13):
+        assert rel(tiles.explicit_run(steps)[0], walk.explicit_run(steps)[0]) <= 1e-12
+    tiles.assemble(pdx.PDX_MODE_STATIC, want_K=False)  # another K: the families' moments are formed again
+    assert rel(tiles.explicit_run(7)[0], walk.explicit_run(7)[0]) <= 1e-12
+    _tiled(tiles, model)
 
 
 def test_fp32_newmark_through_tiles():
     """FP32 vectors with FP64 element arithmetic (large models only), refined: the same displacements as in FP64."""
     model = pdx.Model(_dt(W.box3d(n=65, pd_block=12)))
-    run = [pdx.Context(model).newmark_run(2, pdx.solve_opts(precond=pdx.PDX_PREC_BLOCK_JACOBI, precision=p, tol=1e-10))
-           for p in (pdx.PDX_FP64, pdx.PDX_FP32)]
+    run = []
+    for p in (pdx.PDX_FP64, pdx.PDX_FP32):
+        cx = pdx.Context(model)
+        run.append(cx.newmark_run(2, pdx.solve_opts(precond=pdx.PDX_PREC_BLOCK_JACOBI, precision=p, tol=1e-10)))
     assert run[1][3]["converged"] and run[1][3]["refinements"] > 0
+    _tiled(cx, model)
     for x, y in zip(run[0][:3], run[1][:3]):
         assert rel(y, x) <= 1e-8
 
@@ -159,5 +220,6 @@ def test_newmark_with_beta_zero(n, precision):
     dU = model.values()
     for s in mesh["ebc"]:
         dU[(np.asarray(s["nid"]) - 1) * 3 + s["dof"]] += mesh["dt"] * s.get("vel", 0.0) * bool(s.get("vary", False))
+    _tiled(cx, model)
     F = pdx.Context(model).assemble(pdx.PDX_MODE_NEWMARK, UN=dU)[1]
     assert np.linalg.norm(F - M @ a) <= (1e-8 + 1e-11) * np.linalg.norm(F)

@@ -159,6 +159,7 @@ def test_context_entry_points_reject_a_null_context():
         "pdx_ctx_bonds": (null, ibuf),
         "pdx_local_damage": (null, buf),
         "pdx_explicit_set_form": (null, 0, 0),
+        "pdx_tile_counts": (null, buf),
         "pdx_max_eig": (null, 10, buf),
         "pdx_set_dt": (null, 1e-7),
     }
