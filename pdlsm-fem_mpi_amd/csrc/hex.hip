@@ -115,9 +115,8 @@ void place_elements(const Model &m, const std::vector<unsigned short> &loc, Host
 }  // namespace
 
 // The tiles of a model on the host (nfe_off, nfe_item: per node its FE elements in element order, as
-// FE position * 8 + corner); empty where fewer than min_nodes nodes have hex8 rows
-void hex_tiles_host(const Model &m, const std::vector<int> &nfe_off, const std::vector<int> &nfe_item, long long min_nodes,
-                    HexTilesHost &H) {
+// FE position * 8 + corner); empty where no product would go through them
+void hex_tiles_host(const Model &m, const std::vector<int> &nfe_off, const std::vector<int> &nfe_item, HexTilesHost &H) {
     // nodes whose row is a sum of hex8 elements only
     const std::vector<int> &off = nfe_off;
     auto inc = [&](int j) { return m.fe[nfe_item[j] >> 3]; };
@@ -131,7 +130,19 @@ void hex_tiles_host(const Model &m, const std::vector<int> &nfe_off, const std::
     std::vector<int> nodes;
     for (int k = 0; k < m.nn; k++)
         if (hex[k]) nodes.push_back(k);
-    if (nodes.empty() || (long long)nodes.size() < min_nodes) return;
+    if ((long long)nodes.size() < HEX_MIN_NODES) return;
+    // families of nodes without elements and without boundary terms; the other rows are left to K
+    std::vector<char> edge((size_t)m.nn, 0);
+    for (int p = 0; p < m.npdbe; p++)
+        for (int a = 0; a < 4; a++) edge[m.pdbe[(size_t)p * 4 + a]] = 1;
+    auto by_family = [&](int k) { return m.famid[k] >= 0 && !edge[k] && off[k + 1] == off[k]; };
+    long long n_fam = 0, n_row = 0;
+    for (int k = 0; k < m.nn; k++)
+        if (!hex[k]) (by_family(k) ? n_fam : n_row)++;
+    // no need to build them where even full tiles with the fewest elements would take too long
+    const double limit = HEX_WALK * hex_walk_us(m.adj_off[m.nn]), nh = (double)nodes.size();
+    const double limit32 = m.nn >= HEX_MIN_NODES_F32 ? hex_walk_f32_us(m.adj_off[m.nn]) : 0.0;
+    if (hex_tiles_us(nh / 8, nh / HT_OWN, (double)n_row, (double)n_fam) > std::max(limit, limit32)) return;
     // mean node spacing, from the volume of the elements around the nodes
     double vol = 0.0;
     for (int k : nodes) vol += m.nv[k];
@@ -185,7 +196,10 @@ void hex_tiles_host(const Model &m, const std::vector<int> &nfe_off, const std::
                     }
                     end = k + 1;
                 }
-                if (end == at) break;  // a node of more elements than a tile holds: left to its row of K
+                if (end == at) {  // a node of more elements than a tile holds: left to its row of K
+                    at++;
+                    continue;
+                }
                 // end on a layer of nodes where that keeps most of the tile
                 if (end < last && layer > at && layer < end && layer - at >= (end - at) * 6 / 10) end = layer;
                 // the owned nodes in node order, then the other nodes of their elements as these list them
@@ -248,14 +262,17 @@ void hex_tiles_host(const Model &m, const std::vector<int> &nfe_off, const std::
         std::copy(all[k]->conn.begin(), all[k]->conn.end(), H.conn.begin() + (size_t)H.tile[k].ele0 * 8);
         for (int i = 0; i < all[k]->n_own; i++) owned[all[k]->node[i]] = 1;
     }
-    // families of nodes without elements and without boundary terms, and the rows left to K
-    std::vector<char> edge((size_t)m.nn, 0);
-    for (int p = 0; p < m.npdbe; p++)
-        for (int a = 0; a < 4; a++) edge[m.pdbe[(size_t)p * 4 + a]] = 1;
     for (int k = 0; k < m.nn; k++) {
         if (owned[k]) continue;
-        if (m.famid[k] >= 0 && !edge[k] && off[k + 1] == off[k]) H.fams.push_back(m.famid[k]);
+        if (by_family(k)) H.fams.push_back(m.famid[k]);
         else H.rows.push_back(k);
+    }
+    const double us = hex_tiles_us((double)H.n_ele, (double)all.size(), (double)H.rows.size(), (double)H.fams.size());
+    H.use[0] = us <= limit;
+    H.use[1] = us <= limit32;
+    if (!H.use[0] && !H.use[1]) {
+        H = HexTilesHost();
+        return;
     }
     // each XCD's list: its eighth of the tiles, families and rows, evenly mixed
     const int n[3] = {(int)H.tile.size(), int(H.fams.size() + HEX_FAMS - 1) / HEX_FAMS,
@@ -296,7 +313,7 @@ static int build_hex_tiles(Ctx &c, HexTilesHost &H, std::string &err) {
     PDX_HIP(hipMemcpy(off.data(), c.nfe_off, off.size() * sizeof(int), hipMemcpyDeviceToHost));
     item.resize((size_t)off[c.nn]);
     if (!item.empty()) PDX_HIP(hipMemcpy(item.data(), c.nfe_item, item.size() * sizeof(int), hipMemcpyDeviceToHost));
-    hex_tiles_host(*c.host, off, item, HEX_MIN_NODES, H);
+    hex_tiles_host(*c.host, off, item, H);
     if (H.tile.empty()) return PDX_OK;
     auto *T = new HexTiles();
     c.hex = T;
@@ -305,6 +322,8 @@ static int build_hex_tiles(Ctx &c, HexTilesHost &H, std::string &err) {
     T->n_tile = (int)H.tile.size();
     T->n_row = (int)H.rows.size();
     T->n_ele = H.n_ele;
+    T->use[0] = H.use[0];
+    T->use[1] = H.use[1];
     auto alloc = [&](auto *&dst, size_t n) -> int {
         const hipError_t e = hipMalloc((void **)&dst, std::max<size_t>(n, 1) * sizeof(*dst));
         if (e == hipSuccess) return PDX_OK;
@@ -326,10 +345,10 @@ static int build_hex_tiles(Ctx &c, HexTilesHost &H, std::string &err) {
     return PDX_OK;
 }
 
-int hex_tiles(Ctx &c, const HexTiles *&out, std::string &err) {
-    out = (const HexTiles *)c.hex;
-    if (c.hex_tried) return PDX_OK;
-    if (c.dim == 3 && c.nn >= HEX_MIN_NODES && c.host && c.host->dim == 3) {
+int hex_tiles(Ctx &c, int pi, const HexTiles *&out, std::string &err) {
+    out = nullptr;
+    if (pi && c.nn < HEX_MIN_NODES_F32) return PDX_OK;
+    if (!c.hex_tried && c.dim == 3 && c.nn >= HEX_MIN_NODES && c.host && c.host->dim == 3) {
         HexTilesHost H;
         int rc;
         try {
@@ -345,7 +364,8 @@ int hex_tiles(Ctx &c, const HexTiles *&out, std::string &err) {
         }
     }
     c.hex_tried = true;
-    out = (const HexTiles *)c.hex;
+    const auto *T = (const HexTiles *)c.hex;
+    if (T && T->use[pi]) out = T;
     return PDX_OK;
 }
 

@@ -41,6 +41,7 @@ struct HexTiles {
     int *fams = nullptr;  // families whose rows hold nothing but their bonds, 16 lanes each
     int n_tile = 0, n_row = 0;
     long long n_ele = 0;  // elements of all tiles
+    bool use[2] = {false, false};  // whether products of FP64 / FP32 vectors go through them
 };
 constexpr int HEX_ROWS = HT_THREADS / 64;  // rows of a block
 constexpr int HEX_FAMS = HT_THREADS / 16;  // families of a block
@@ -50,9 +51,9 @@ struct HexTilesHost {
     std::vector<int> nodes, rows, fams;
     std::vector<unsigned short> conn;
     long long n_ele = 0;
+    bool use[2] = {false, false};  // as in HexTiles
 };
-void hex_tiles_host(const Model &m, const std::vector<int> &nfe_off, const std::vector<int> &nfe_item, long long min_nodes,
-                    HexTilesHost &H);
+void hex_tiles_host(const Model &m, const std::vector<int> &nfe_off, const std::vector<int> &nfe_item, HexTilesHost &H);
 
 // Fewer nodes than this keep their rows in K: their tiles leave CUs idle through the several
 // microseconds of one tile (explicit step at 24^3 nodes: 8.5 us against 7.4 for the walk of K; at
@@ -64,9 +65,33 @@ constexpr long long HEX_MIN_NODES = 20480;
 // box: 48^3 107 against 110, 60^3 156 against 169, 80^3 409 against 349.
 constexpr int HEX_MIN_NODES_F32 = 262144;
 
-// The context's tiles (built on first use), or null where the products go through K: 2D models and
-// models with few nodes whose rows are hex8 sums (HEX_MIN_NODES)
-int hex_tiles(Ctx &c, const HexTiles *&out, std::string &err);
+// Microseconds of a product through the tiles and of one that walks K, as sums over what they consist
+// of.  Least squares over explicit steps of 35 models of 24,000 to 720,000 nodes: cubes, plates of 2 to
+// 6 node layers, bars, boxes with spacings up to 1 : 100, boxes partly of tetrahedra, PD blocks of 41^3
+// and 49^3 nodes.  The tiles' sum is within 17% of each, the walk's within 20%.  A tile of a cube holds
+// 143 nodes and an element is computed 1.6 times; at a spacing of 1 : 10 it is 50 and 3.8, at 1 : 100 19
+// and 7.3.  A row left to K costs a wavefront that reads it unmirrored.
+inline double hex_tiles_us(double elements, double tiles, double rows, double families) {
+    return 6.0 + 5.7e-5 * elements + 5.9e-3 * tiles + 1.5e-3 * rows + 1.4e-3 * families;
+}
+inline double hex_walk_us(double blocks) { return 3.3 + 1.11e-5 * blocks; }
+// FP32 blocks in mirrored storage, from HEX_MIN_NODES_F32 nodes on: up to some 9M blocks stay in the
+// Infinity Cache (15 models of 216,000 to 1,080,000 nodes, within 10%)
+inline double hex_walk_f32_us(double blocks) {
+    return blocks <= 9e6 ? 7.0e-6 * blocks : 63.0 + 1.45e-5 * (blocks - 9e6);
+}
+// FP64 products go through the tiles up to this multiple of the walk's sum, FP32 products up to the walk's
+// own: on these models that is the faster way, or one within 3% of it.  FP64 steps through the tiles
+// against the walk: 60^3 35 and 62 us, plate of 400 x 400 x 4 87 and 204, bar 5 x 5 x 8000 21 and 41; but
+// 300 x 300 x 2 52 and 38, 60^3 with a spacing of 1 : 10 70 and 62, of 1 : 100 148 and 62, with a fifth of
+// tetrahedra 95 and 59, a tenth of them spread out 216 and 62.  FP32: 80^3 72 and 113, 600 x 600 x 2 192
+// and 116, 70^3 with a spacing of 1 : 3 55 and 63, of 1 : 5 70 and 62.
+constexpr double HEX_WALK = 1.1;
+
+// The context's tiles (built on first use) for products of vectors of precision index pi (0 FP64, 1 FP32),
+// or null where these walk K: 2D models, models with few nodes whose rows are hex8 sums (HEX_MIN_NODES,
+// HEX_MIN_NODES_F32), and those whose tiles would take longer (HEX_WALK)
+int hex_tiles(Ctx &c, int pi, const HexTiles *&out, std::string &err);
 void free_hex_tiles(Ctx &c);
 
 // lane l ^ 1's value

@@ -1851,8 +1851,8 @@ static int setup_precond(Ctx &c, const double *K64, const pdx_solve_opts &o, Kry
 // the blocks; a solve whose FP32 products walk them forms its few FP64 residuals from them too)
 static int product_tiles(Ctx &c, int prec, const HexTiles *&ht, std::string &err) {
     ht = nullptr;
-    if (c.dim != 3 || (prec == PDX_FP32 && c.nn < HEX_MIN_NODES_F32)) return PDX_OK;
-    if (int rc = hex_tiles(c, ht, err)) return rc;
+    if (c.dim != 3) return PDX_OK;
+    if (int rc = hex_tiles(c, prec == PDX_FP32 ? 1 : 0, ht, err)) return rc;
     return ht && ht->n_fam ? dev_family_moments(c, err) : PDX_OK;
 }
 

@@ -459,8 +459,8 @@ static void launch_explicit_any(Ctx &c, int prec, int variant, const double *Un,
 // (a form set by the caller, or no tiles for this model)
 static int step_tiles(Ctx &c, int pi, const HexTiles *&ht, std::string &err) {
     ht = nullptr;
-    if (c.tune_explicit[pi] >= 0 || (pi && c.nn < HEX_MIN_NODES_F32)) return PDX_OK;
-    return hex_tiles(c, ht, err);
+    if (c.tune_explicit[pi] >= 0) return PDX_OK;
+    return hex_tiles(c, pi, ht, err);
 }
 
 template <bool FO>
