@@ -413,8 +413,9 @@ int pdx_last_timing(pdx_ctx *c, double *total_ms, double *per_step_ms);
  * 20-23); all 0 before the first step)
  * and its timings of the PDX_EXPLICIT_FORMS forms (ms per step).  A context of a large 3D model steps
  * without walking most of K (rows of hex8 nodes from the elements, of interior PD nodes from their
- * families) while no form is set: the forms are then timed when this is called, and the fastest is
- * reported, not used */
+ * families) while no form is set, and a consistent-mass step has one form: after such steps the forms are
+ * timed at the first call of this, which then allocates what they read, and the fastest is reported, not
+ * used */
 #define PDX_EXPLICIT_FORMS 24
 int pdx_explicit_tuning(pdx_ctx *c, int precision, int *lanes, int *nontemporal, int *xcd_order, int *row_soa,
                         int *col_classes, int *mirrored, int *alternating, int *form,

@@ -176,7 +176,8 @@ struct Ctx {
     // allocated and freed with the tiles
     double *mom_w = nullptr, *mom_T = nullptr;
     long long mom_gen = -1;
-    int tune_seen[2] = {-1, -1};  // form the tuner found for a context that steps through the tiles
+    bool stepped[2] = {false, false};  // explicit steps of this precision were run
+    int tune_seen[2] = {-1, -1};  // form the tuner found for a context whose steps use none
 
     // scratch for Krylov
     std::vector<DevBuf> scratch;

@@ -608,7 +608,7 @@ static int explicit_operators(Ctx &c, int prec, bool lumped, std::string &err) {
     if (ht) {
         if (ht->n_fam)
             if (int e = dev_family_moments(c, err)) return e;
-    } else {
+    } else if (lumped) {  // the consistent-mass step reads K itself
         if (int e = ensure_Ks(c, prec, err)) return e;
         if (int e = ensure_Kown(c, prec, err)) return e;
     }
@@ -690,8 +690,10 @@ int dev_explicit_dofvals(Ctx &c, const double **out, std::string &err) {
     return PDX_OK;
 }
 
-int explicit_tune_if_needed(Ctx &c, int prec, std::string &err) {
+int explicit_tune_if_needed(Ctx &c, int prec, bool lumped, std::string &err) {
     const int pi = prec == PDX_FP32 ? 1 : 0;
+    c.stepped[pi] = true;
+    if (!lumped) return PDX_OK;  // the consistent-mass step has one form and uses no tiles
     const HexTiles *ht = nullptr;
     int rc = step_tiles(c, pi, ht, err);
     if (rc || ht || c.tune_explicit[pi] >= 0) return rc;
@@ -701,13 +703,13 @@ int explicit_tune_if_needed(Ctx &c, int prec, std::string &err) {
     return rc;
 }
 
-// What pdx_explicit_tuning reports for a context that steps through the tiles: the fastest K form
-// for its current state, timed when first asked for (the steps stay on the tiles)
+// What pdx_explicit_tuning reports for a context whose steps of this precision use none of the forms (through the
+// tiles, or consistent mass): the fastest form for its current state, timed when first asked for
 int explicit_tune_seen(Ctx &c, int pi, std::string &err) {
-    if (c.tune_explicit[pi] >= 0 || c.tune_seen[pi] >= 0 || !c.hex || c.steps_done < 0) return PDX_OK;
+    if (c.tune_explicit[pi] >= 0 || c.tune_seen[pi] >= 0 || !c.stepped[pi] || c.steps_done < 0) return PDX_OK;
     const int prec = pi ? PDX_FP32 : PDX_FP64;
-    if (!c.K_valid) return PDX_OK;
     int rc;
+    if (!c.K_valid && (rc = dev_assemble_K(c, err))) return rc;
     if (!c.mlump_valid && (rc = dev_lumped_mass(c, err))) return rc;
     if (pi && (rc = ensure_K32(c, err))) return rc;
     if ((rc = ensure_Ks(c, prec, err)) || (rc = ensure_Kown(c, prec, err)) || (rc = tune_explicit(c, pi, err))) return rc;
@@ -759,7 +761,7 @@ int dev_explicit_steps(Ctx &c, int nsteps, int prec, int use_graph, bool lumped,
     if (e) return e;
     if (startup && after_step && (e = after_step(err))) return e;
     if (nsteps == 0) return PDX_OK;  // the start-up step only
-    if ((e = explicit_tune_if_needed(c, prec, err))) return e;
+    if ((e = explicit_tune_if_needed(c, prec, lumped, err))) return e;
     const int period = kExplicitPeriod;
     const bool replay = lumped && !after_step && use_graph && nsteps >= period;
     // the graph is captured and instantiated before the timed region

@@ -44,3 +44,19 @@ def test_mass_product_trajectory(name):
     u1, up1 = pdx.Context(pdx.Model(mesh)).explicit_run(12)
     assert np.abs(u0).max() > 0
     assert rel(u1, u0) <= 1e-10 and rel(up1, up0) <= 1e-10, (rel(u1, u0), rel(up1, up0))
+
+
+def test_consistent_steps_build_no_tiles_and_time_no_forms():
+    """A size at which lumped steps go through the element tiles: the consistent-mass step walks K in its one form, so
+    it builds none.  The tuning is timed when it is asked for, for the precision that was stepped only."""
+    mesh = W.box3d(n=30, pd_block=8)
+    mesh["lumped_mass"] = False
+    mesh["dt"] = 2e-8
+    cx = pdx.Context(pdx.Model(mesh))
+    assert cx.explicit_tuning_full(pdx.PDX_FP64)[8] == -1
+    u = cx.explicit_run(3)[0]
+    assert not any(cx.tile_counts().values())
+    assert cx.explicit_tuning_full(pdx.PDX_FP32)[8] == -1 and not cx.explicit_tuning_full(pdx.PDX_FP32)[6].any()
+    full = cx.explicit_tuning_full(pdx.PDX_FP64)
+    assert 0 <= full[8] < pdx.EXPLICIT_FORMS and (full[6] > 0).all()
+    assert np.array_equal(cx.explicit_run(0)[0], u)
