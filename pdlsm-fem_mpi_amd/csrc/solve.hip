@@ -132,7 +132,6 @@ __global__ void __launch_bounds__(256) k_explicit(const int *rows_s, int ns, int
 // FP32: K is 330 MB (196 MB) per step there, while the elements are 8.6M FP64 wavefront instructions (15 us at the full rate) on some 60 MB.  Bound by
 // those two one after the other: two workgroups of 198 registers fit a CU, and the ones in flight load
 // together and calculate together.
-template <bool FO>
 __global__ void __launch_bounds__(HT_THREADS, HT_WAVES) k_explicit_hex(
     HexTiles ht, MomentArgs ma, double lam8, double mu8, const int *adj_off, const int *adj, const double *K,
     const double *x, const double *Un, const double *Unm1, double *Unp1, const double *m, const double *f_unit, int n_nbc,
@@ -151,8 +150,8 @@ __global__ void __launch_bounds__(HT_THREADS, HT_WAVES) k_explicit_hex(
         Dof d;
         d.o = (size_t)r * 3 + i;
         d.eq = eq[d.o];
-        d.m = FO ? 1.0 : m[d.o];
-        d.unm1 = FO ? 0.0 : Unm1[d.o];
+        d.m = m[d.o];
+        d.unm1 = Unm1[d.o];
         d.fext = 0.0;
         for (int s = 0; s < n_nbc; s++) d.fext = d.fext + nbc_cur[s] * f_unit[(size_t)s * nn * 3 + d.o];
         return d;
@@ -160,8 +159,7 @@ __global__ void __launch_bounds__(HT_THREADS, HT_WAVES) k_explicit_hex(
     auto update = [&](const Dof &d, double un, double v) {
         const double F = d.fext - v;
         double y;
-        if (d.eq < 0) y = FO ? 0.0 : un + ebc_inc[presc_set[d.o]];
-        else if (FO) y = F;
+        if (d.eq < 0) y = un + ebc_inc[presc_set[d.o]];
         else if (startup) y = F / d.m * (0.5 * dt * dt) + un;
         else y = un * 2.0 + dt * dt * F / d.m - d.unm1;
         Unp1[d.o] = y;
@@ -463,11 +461,10 @@ static int step_tiles(Ctx &c, int pi, const HexTiles *&ht, std::string &err) {
     return hex_tiles(c, pi, ht, err);
 }
 
-template <bool FO>
 static void launch_explicit_hex(Ctx &c, const HexTiles &ht, const double *Un, const double *Unm1, double *Unp1,
                                 const double *nbc_cur, double *nbc_next, int startup) {
     c.hex_products++;
-    k_explicit_hex<FO><<<ht.n_work, HT_THREADS, 0, c.stream>>>(
+    k_explicit_hex<<<ht.n_work, HT_THREADS, 0, c.stream>>>(
         ht, moment_args(c), c.lambda / 8, c.mu / 8, c.adj_off, c.adj, c.K, c.x, Un, Unm1, Unp1, c.mlump, c.f_unit, c.n_nbc, c.nn,
         nbc_cur, nbc_next, c.d_nbc_vel, c.eq, c.presc_set, c.d_ebc_vel, c.dt, startup);
 }
@@ -518,7 +515,7 @@ static void explicit_step(Ctx &c, int prec, int startup) {
     std::string unused;  // the tiles, if any, were built by explicit_operators
     step_tiles(c, prec == PDX_FP32 ? 1 : 0, ht, unused);
     if (ht)
-        launch_explicit_hex<false>(c, *ht, Un, Unm1, Unp1, nbc_cur, nbc_next, startup);
+        launch_explicit_hex(c, *ht, Un, Unm1, Unp1, nbc_cur, nbc_next, startup);
     else
         launch_explicit_any(c, prec, std::max(c.tune_explicit[prec == PDX_FP32 ? 1 : 0], 0), Un, Unm1, Unp1, nbc_cur,
                             nbc_next, startup, s);
