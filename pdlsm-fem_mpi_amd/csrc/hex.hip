@@ -1,8 +1,10 @@
 // Node tiles for the products with hex8 elements without their K blocks (hex.hpp): host set-up.
 #include <hip/hip_runtime.h>
+#include <omp.h>
 
 #include <algorithm>
 #include <array>
+#include <atomic>
 #include <bitset>
 #include <cmath>
 #include <cstring>
@@ -19,8 +21,27 @@ namespace {
 // one tile under construction on the host
 struct HostTile {
     int n_own = 0;
-    std::vector<int> node, ele, place;  // place: the elements in groups of HT_GROUP, -1 for an empty place
-    std::vector<unsigned short> conn;
+    std::vector<int> node, ele, place;  // place: positions in ele in groups of HT_GROUP, -1 for an empty place
+    std::vector<unsigned short> corner, conn;  // local numbers of the corners, by element and by place
+};
+
+// Out of memory inside a parallel loop: an exception must not leave the loop's body, so the first one is noted and
+// thrown again behind the loop
+class LoopMemory {
+    std::atomic<bool> out{false};
+
+public:
+    template <typename F>
+    void body(F &&f) {
+        try {
+            f();
+        } catch (const std::bad_alloc &) {
+            out = true;
+        }
+    }
+    void check() const {
+        if (out) throw std::bad_alloc();
+    }
 };
 
 // v[b, e) by coordinate, then node
@@ -54,8 +75,10 @@ void sort_along_parallel(std::vector<int> &v, const double *x, int axis) {
     std::vector<int> out(n);
     for (size_t i = 0; i < n; i++) out[fill[at[i]]++] = v[i];
     v.swap(out);
+    LoopMemory mem;
 #pragma omp parallel for schedule(dynamic, 8)
-    for (int i = 0; i < NB; i++) sort_along(v, off[i], off[i + 1], x, axis);
+    for (int i = 0; i < NB; i++) mem.body([&] { sort_along(v, off[i], off[i + 1], x, axis); });
+    mem.check();
 }
 
 // Nodes in slabs along x, the slabs in columns along y, each about `w` node spacings wide, the cuts
@@ -85,16 +108,15 @@ void cut_even(const std::vector<int> &v, size_t b, size_t e, const double *x, in
 }
 
 // Elements into groups of HT_GROUP, in order, none beside another with the same node in the same
-// corner (two elements of a consistently numbered mesh never are); loc: local number of a node
-void place_elements(const Model &m, const std::vector<unsigned short> &loc, HostTile &t) {
+// corner (two elements of a consistently numbered mesh never are)
+void place_elements(HostTile &t) {
     using Used = std::bitset<HT_NODES>;
     std::vector<std::array<Used, 8>> used;  // nodes in each corner of each group
     std::vector<int> count;                 // elements of each group
     size_t first = 0;                       // the first group with a place left
     t.place.clear();
-    for (int e : t.ele) {
-        unsigned short l[8];
-        for (int a = 0; a < 8; a++) l[a] = loc[m.econ[(size_t)e * 8 + a]];
+    for (int e = 0; e < (int)t.ele.size(); e++) {
+        const unsigned short *l = &t.corner[(size_t)e * 8];
         while (first < count.size() && count[first] == HT_GROUP) first++;
         size_t g = first;
         for (; g < count.size(); g++) {
@@ -152,23 +174,35 @@ void hex_tiles_host(const Model &m, const std::vector<int> &nfe_off, const std::
     cut_even(nodes, 0, nodes.size(), m.x.data(), 0, width, xs);
     // columns: the slabs cut along y, each sorted along z
     std::vector<std::vector<size_t>> ys(xs.size() - 1);
+    LoopMemory mem;
 #pragma omp parallel for schedule(dynamic, 1)
-    for (int s = 0; s < (int)xs.size() - 1; s++) {
-        sort_along(nodes, xs[s], xs[s + 1], m.x.data(), 1);
-        cut_even(nodes, xs[s], xs[s + 1], m.x.data(), 1, width, ys[s]);
-    }
+    for (int s = 0; s < (int)xs.size() - 1; s++)
+        mem.body([&] {
+            sort_along(nodes, xs[s], xs[s + 1], m.x.data(), 1);
+            cut_even(nodes, xs[s], xs[s + 1], m.x.data(), 1, width, ys[s]);
+        });
+    mem.check();
     std::vector<std::pair<size_t, size_t>> column;
     for (auto &y : ys)
         for (size_t q = 0; q + 1 < y.size(); q++) column.push_back({y[q], y[q + 1]});
     std::vector<std::vector<HostTile>> per_column(column.size());
-#pragma omp parallel
+    // a thread's marks are 10 bytes per node and element: as many threads as a gigabyte holds
+    const double marks = 4.0 * m.ne + 6.0 * m.nn;
+    const int threads = (int)std::max(1.0, std::min((double)omp_get_max_threads(), 1e9 / marks));
+#pragma omp parallel num_threads(threads)
     {
         // number of the last tile that took the element / node
-        std::vector<int> in_e((size_t)m.ne, -1), in_n((size_t)m.nn, -1);
-        std::vector<unsigned short> loc((size_t)m.nn);  // local number of a node of the current tile
+        std::vector<int> in_e, in_n;
+        std::vector<unsigned short> loc;  // local number of a node of the current tile
+        mem.body([&] {
+            in_e.assign((size_t)m.ne, -1);
+            in_n.assign((size_t)m.nn, -1);
+            loc.resize((size_t)m.nn);
+        });
         int serial = 0;
 #pragma omp for schedule(dynamic, 1)
-        for (int q = 0; q < (int)column.size(); q++) {
+        for (int q = 0; q < (int)column.size(); q++) mem.body([&] {
+            if (loc.size() != (size_t)m.nn) return;  // this thread's marks did not fit
             const size_t last = column[q].second;
             sort_along(nodes, column[q].first, last, m.x.data(), 2);
             size_t at = column[q].first;
@@ -206,9 +240,12 @@ void hex_tiles_host(const Model &m, const std::vector<int> &nfe_off, const std::
                 t.node.assign(nodes.begin() + at, nodes.begin() + end);
                 std::sort(t.node.begin(), t.node.end());
                 t.n_own = int(t.node.size());
+                t.corner.reserve(HT_ELE * 8);
                 serial++;
-                for (int nd : t.node) {
+                for (int i = 0; i < t.n_own; i++) {
+                    const int nd = t.node[i];
                     in_n[nd] = serial;
+                    loc[nd] = (unsigned short)i;
                     for (int j = off[nd]; j < off[nd + 1]; j++) {
                         const int e = inc(j);
                         if (in_e[e] == serial) continue;
@@ -220,20 +257,24 @@ void hex_tiles_host(const Model &m, const std::vector<int> &nfe_off, const std::
                 for (int e : t.ele)
                     for (int a = 0; a < 8; a++) {
                         const int v = m.econ[(size_t)e * 8 + a];
-                        if (in_n[v] == serial) continue;
-                        in_n[v] = serial;
-                        t.node.push_back(v);
+                        if (in_n[v] != serial) {
+                            in_n[v] = serial;
+                            loc[v] = (unsigned short)t.node.size();
+                            t.node.push_back(v);
+                        }
+                        t.corner.push_back(loc[v]);
                     }
-                for (size_t i = 0; i < t.node.size(); i++) loc[t.node[i]] = (unsigned short)i;
-                place_elements(m, loc, t);
+                place_elements(t);
                 t.conn.assign(t.place.size() * 8, 0xffff);
                 for (size_t i = 0; i < t.place.size(); i++)
-                    for (int a = 0; a < 8 && t.place[i] >= 0; a++) t.conn[i * 8 + a] = loc[m.econ[(size_t)t.place[i] * 8 + a]];
+                    if (t.place[i] >= 0) std::copy_n(&t.corner[(size_t)t.place[i] * 8], 8, &t.conn[i * 8]);
+                t.corner = std::vector<unsigned short>();
                 per_column[q].push_back(std::move(t));
                 at = end;
             }
-        }
+        });
     }
+    mem.check();
     // flat arrays
     std::vector<const HostTile *> all;
     for (auto &col : per_column)

@@ -1,7 +1,7 @@
 """Host half of the element tiles (csrc/hex.hip) on the CPU: the file is compiled for the host with a runtime whose
 allocations are host memory and fail on demand.
 
-A context whose tile arrays do not fit walks K: each allocation failing in turn, the call succeeds without tiles,
+A context whose tile arrays do not fit (on the device or the host) walks K: each device allocation failing in turn, the call succeeds without tiles,
 nothing is left allocated, a second call does not try (or read) again, and a new context builds the same tiles as
 one that never failed.
 
@@ -26,6 +26,13 @@ RUNTIME = r"""
 #include "setup.hpp"
 
 static int g_fail_at = -1, g_calls = 0;
+static std::atomic<long> g_new_calls{0}, g_new_fail_at{-1};
+void *operator new(size_t n) {
+    if (g_new_calls++ == g_new_fail_at) throw std::bad_alloc();
+    return std::malloc(n ? n : 1);
+}
+void operator delete(void *p) noexcept { std::free(p); }
+void operator delete(void *p, size_t) noexcept { std::free(p); }
 static std::set<void *> g_live;
 extern "C" {
 hipError_t hipMalloc(void **p, size_t n) {
@@ -177,7 +184,22 @@ int main() {
         if (hex_tiles(n.c, 0, t, err) || !t || t->n_work != work) return 5;
         free_hex_tiles(n.c);
     }
-    std::printf("%d allocations, %d blocks\n", calls, work);
+    // host memory too, on whichever thread it runs out
+    long news = 0, failed = 0;
+    for (long at = 0;; at += 1 + at / 3) {
+        Host h(m);
+        g_new_calls = 0;
+        g_new_fail_at = at;
+        const int rc = hex_tiles(h.c, 0, t, err);
+        g_new_fail_at = -1;
+        if (rc || !t != !h.c.hex || (!t && !g_live.empty())) return std::printf("host allocation %ld\n", at), 7;
+        news = g_new_calls;
+        failed += !t;
+        free_hex_tiles(h.c);
+        if (at > 2 * news) break;
+    }
+    if (failed < 10) return 8;
+    std::printf("%d allocations, %d blocks; %ld host allocations, %ld failed\n", calls, work, news, failed);
     return g_live.empty() ? 0 : 6;
 }
 """
