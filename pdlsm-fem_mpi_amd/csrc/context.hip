@@ -339,6 +339,10 @@ int ctx_build(const Model &m, int device, Ctx *&out, std::string &err) {
                 if (!((pd_bits[(size_t)q >> 3] >> (q & 7)) & 1) && fcnt[q + 1] == fcnt[q]) bare++;
             c->k_needs_fill = bare > 0;
         }
+        if (D == 3 && m.nn >= HEX_MIN_NODES) {
+            c->nfe_off_host = std::move(cnt);
+            c->nfe_item_host = std::move(item);
+        }
         // all elements (lumped mass)
         std::vector<int> acnt(m.nn + 1, 0);
         for (int e = 0; e < m.ne; e++)

@@ -171,6 +171,9 @@ struct Ctx {
     void *hex = nullptr;
     bool hex_tried = false;
     long long hex_products = 0;  // launched or captured so far
+    // nfe_off, nfe_item on the host until the tiles are built or refused (3D, HEX_MIN_NODES nodes and more): moved
+    // here by the set-up; to fetch them from the device adds 2 ms to the first step of a 60^3 box
+    std::vector<int> nfe_off_host, nfe_item_host;
     // PD rows formed from the moments of their families (hex.hpp): bond weights [members] and the
     // second-order rows of the inverse shape tensors [nfam * 54], for the K of generation mom_gen;
     // allocated and freed with the tiles

@@ -347,14 +347,9 @@ void hex_tiles_host(const Model &m, const std::vector<int> &nfe_off, const std::
 }
 
 // The device arrays of the tiles, and those of the family moments, which only products through the
-// tiles read.  The incidence lists come back from the device (7 MB of a 60^3 box), so no copy of them
-// waits on the host.
+// tiles read
 static int build_hex_tiles(Ctx &c, HexTilesHost &H, std::string &err) {
-    std::vector<int> off((size_t)c.nn + 1), item;
-    PDX_HIP(hipMemcpy(off.data(), c.nfe_off, off.size() * sizeof(int), hipMemcpyDeviceToHost));
-    item.resize((size_t)off[c.nn]);
-    if (!item.empty()) PDX_HIP(hipMemcpy(item.data(), c.nfe_item, item.size() * sizeof(int), hipMemcpyDeviceToHost));
-    hex_tiles_host(*c.host, off, item, H);
+    hex_tiles_host(*c.host, c.nfe_off_host, c.nfe_item_host, H);
     if (H.tile.empty()) return PDX_OK;
     auto *T = new HexTiles();
     c.hex = T;
@@ -389,7 +384,7 @@ static int build_hex_tiles(Ctx &c, HexTilesHost &H, std::string &err) {
 int hex_tiles(Ctx &c, int pi, const HexTiles *&out, std::string &err) {
     out = nullptr;
     if (pi && c.nn < HEX_MIN_NODES_F32) return PDX_OK;
-    if (!c.hex_tried && c.dim == 3 && c.nn >= HEX_MIN_NODES && c.host && c.host->dim == 3) {
+    if (!c.hex_tried && c.dim == 3 && c.host && c.host->dim == 3 && !c.nfe_off_host.empty()) {
         HexTilesHost H;
         int rc;
         try {
@@ -404,7 +399,11 @@ int hex_tiles(Ctx &c, int pi, const HexTiles *&out, std::string &err) {
             err.clear();
         }
     }
-    c.hex_tried = true;
+    if (!c.hex_tried) {  // built, or never to be: the lists have served
+        c.hex_tried = true;
+        c.nfe_off_host = std::vector<int>();
+        c.nfe_item_host = std::vector<int>();
+    }
     const auto *T = (const HexTiles *)c.hex;
     if (T && T->use[pi]) out = T;
     return PDX_OK;

@@ -153,8 +153,8 @@ struct Host {
         c.nn = m.nn;
         c.nfam = m.nfam;
         c.host = &m;
-        c.nfe_off = off.data();
-        c.nfe_item = item.data();
+        c.nfe_off_host = off;
+        c.nfe_item_host = item;
     }
 };
 """
