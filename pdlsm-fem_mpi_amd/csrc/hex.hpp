@@ -56,12 +56,12 @@ struct HexTilesHost {
 void hex_tiles_host(const Model &m, const std::vector<int> &nfe_off, const std::vector<int> &nfe_item, HexTilesHost &H);
 
 // Fewer nodes than this keep their rows in K: their tiles leave CUs idle through the several
-// microseconds of one tile (explicit step at 24^3 nodes: 8.5 us against 7.4 for the walk of K; at
-// 31^3: 11.8 against 13.0)
+// microseconds of one tile (explicit step at 24^3 nodes, 8^3 of them PD: 8.7 us against 6.8 for the walk of
+// K; at 31^3, 10^3 PD: 12.2 against 12.7)
 constexpr long long HEX_MIN_NODES = 20480;
 // FP32 products walk the blocks up to this many nodes: 4-byte blocks stay in the 256 MB Infinity Cache
-// so long.  Explicit step: 31^3 nodes 9.5 us against 11.7 through the tiles; 60^3: 44.8 against 44.0,
-// for a longer first call; 66^3: 58.3 against 55.8; 80^3: 124 against 86.  Newmark iteration, penny
+// so long.  Explicit step: 31^3 nodes 9.3 us against 12.2 through the tiles; 60^3: 44.6 against 44.5,
+// for a longer first call; 66^3: 58.8 against 55.6; 80^3: 120 against 81.  Newmark iteration, penny
 // box: 48^3 107 against 110, 60^3 156 against 169, 80^3 409 against 349.
 constexpr int HEX_MIN_NODES_F32 = 262144;
 
@@ -70,9 +70,11 @@ constexpr int HEX_MIN_NODES_F32 = 262144;
 // 6 node layers, bars, boxes with spacings up to 1 : 100, boxes partly of tetrahedra, PD blocks of 41^3
 // and 49^3 nodes.  The tiles' sum is within 17% of each, the walk's within 20%.  A tile of a cube holds
 // 143 nodes and an element is computed 1.6 times; at a spacing of 1 : 10 it is 50 and 3.8, at 1 : 100 19
-// and 7.3.  A row left to K costs a wavefront that reads it unmirrored.
+// and 7.3.  A row left to K costs a wavefront that reads it unmirrored.  A family's chain of loads shows in
+// a short launch: 28^3 nodes 9.0 us against 9.3 for the walk, with 9^3 PD nodes 11.5 against 9.7; 33^3 with
+// 8^3 12.5 against 13.6, 48^3 with 10^3 24.9 against 32.9.
 inline double hex_tiles_us(double elements, double tiles, double rows, double families) {
-    return 6.0 + 5.7e-5 * elements + 5.9e-3 * tiles + 1.5e-3 * rows + 1.4e-3 * families;
+    return 6.0 + 5.7e-5 * elements + 5.9e-3 * tiles + 1.5e-3 * rows + 1.4e-3 * families + (families > 0.0 ? 1.8 : 0.0);
 }
 inline double hex_walk_us(double blocks) { return 3.3 + 1.11e-5 * blocks; }
 // FP32 blocks in mirrored storage, from HEX_MIN_NODES_F32 nodes on: up to some 9M blocks stay in the

@@ -240,7 +240,7 @@ int main() {
     struct { const char *name; int nx, ny, nz; double hz; int pd, tets; bool want; } c[] = {
         {"cube", 30, 30, 30, s, 8, 0, true},          {"plate of 4 layers", 80, 80, 4, s, 0, 0, true},
         {"bar", 5, 5, 1000, s, 0, 0, true},           {"few nodes", 26, 26, 30, s, 0, 0, false},
-        {"plate of 2 layers", 120, 120, 2, s, 0, 0, false}, {"spacing 100 : 1", 31, 31, 31, s / 100, 0, 0, false},
+        {"small with PD", 28, 28, 28, s, 10, 0, false}, {"plate of 2 layers", 120, 120, 2, s, 0, 0, false}, {"spacing 100 : 1", 31, 31, 31, s / 100, 0, 0, false},
         {"a fifth tetrahedra", 33, 33, 33, s, 0, 6, false},
         {"mostly tetrahedra", 30, 30, 90, s, 0, 60, false}};
     for (auto &q : c) {
