@@ -92,17 +92,11 @@ def step_bytes(m, nblk, prec, col_classes=None, n_own=None):
     return vals + cols + (m.nn + 1) * 4 + m.nn * d * 8 + m.nn * d * (8 * 4 + 8)
 
 
-def through_tiles(m, prec):
-    """Whether the explicit step forms the rows of the hex8 nodes from the elements and those of the interior
-    PD nodes from their families' moments instead of walking K (the library's rule on sizes)."""
-    fe_nodes = m.nn - m.nfam
-    return m.dim == 3 and fe_nodes >= 20480 and (prec == 0 or m.nn >= 262144)
-
-
 def tile_step_work(m):
-    """(bytes, FP64 flops) of one such step: coordinates, element nodes, bond weights and members once, and
-    per DOF u_n, u_{n-1}, m, unit traction force and u_{n+1}; per element two planes of four Gauss points
-    (150 multiply-adds, adds and multiplies each, counted with the plane's interpolations as 1,200 flops)."""
+    """(bytes, FP64 flops) of one step through the element tiles: coordinates, element nodes, bond weights and members
+    once, and per DOF u_n, u_{n-1}, m, unit traction force and u_{n+1}; per element, each counted once (the tiles compute
+    those between two of them in both), two planes of four Gauss points (150 multiply-adds, adds and multiplies each,
+    counted with the plane's interpolations as 1,200 flops)."""
     nfe = int((m.nodes()["algo"] == 2).sum())
     return m.nn * 24 + nfe * 32 + m.nmem * 12 + m.nn * m.dim * 40, nfe * 2 * 1200 + m.nmem * 70
 
@@ -698,16 +692,17 @@ def main():
                       "column_classes": {"classes": classes[0], "offsets": classes[1]},
                       "mirrored_storage": {"own_blocks": n_own, "blocks": nblk},
                       "scalar_csr_bytes_per_step": scalar_csr_step_bytes(model, prec)}
-        if through_tiles(model, prec):
+        tiles = ctxs[prec].tile_counts()
+        if tiles["products"]:  # the steps went through the element tiles instead of walking K
             nbytes, flops = tile_step_work(model)
             sec = res[prec]["step_ms"] * 1e-3
             k_walk = {k: roof[prec][k] for k in ("form", "tuner_ms_per_form", "column_classes", "mirrored_storage",
                                                  "scalar_csr_bytes_per_step")}
             roof[prec] = {"bound": "fp64_vector", "achieved": flops / sec / 1e12, "peak": FP64_PEAK / 1e12,
-                          "unit": "TFLOP/s", "frac": flops / sec / FP64_PEAK, "traffic": None,
-                          "kernel": f"pdx::k_explicit_hex<{ty}, false> (element and family products + central-difference "
-                                    "update)",
-                          "bytes_per_launch": nbytes, "hbm_frac": nbytes / sec / HBM_PEAK, "walk_of_K": k_walk}
+                          "unit": "TFLOP/s", "frac": flops / sec / FP64_PEAK,
+                          "traffic": measured_traffic("pdx::k_explicit_hex") if args.n == 60 else None,
+                          "kernel": "pdx::k_explicit_hex (element and family products + central-difference update)",
+                          "tiles": tiles, "bytes_per_launch": nbytes, "hbm_frac": nbytes / sec / HBM_PEAK, "walk_of_K": k_walk}
     # the headline is the reference's precision (FP64 values, FP64 accumulation, FP64 state);
     # the FP32-force / FP64-state figure and its drift against FP64 follow as secondary keys
     head = {"metric": METRIC, "value": res[0]["dofs"], "unit": "DOF-steps/s", "n_gpus": 1, "steps": args.steps,

@@ -150,8 +150,9 @@ __global__ void __launch_bounds__(256) k_spmv_dot(const int *rows_s, int ns, int
 // hex8 nodes come from the elements, those of the interior PD nodes from their families' moments
 // (hex.hpp), the others from the operator's FP64 blocks K, a wavefront each.  FP64
 // arithmetic for FP32 vectors too.  Each block writes its dot partials to bp0 / bp1 at its own slot.
-// 80^3 penny box, K_eff: 92 us per product where the walk of its blocks takes 202 in FP64 and 120 in
-// FP32 (mirrored storage).  Bound as the explicit step's kernel is.
+// 80^3 penny box, K_eff: 90 us per product for FP64 vectors, 103 for FP32 ones (traced averages), where the
+// walk of its blocks takes 202 and 120 (mirrored storage); 100^3: 209 and 201 against 398 and 258.  Bound as
+// the explicit step's kernel is.
 template <typename V, bool MASS>
 __global__ void __launch_bounds__(HT_THREADS, HT_WAVES) k_spmv_hex(
     HexTiles ht, MomentArgs ma, double ks, double lam8, double mu8, double rho8, double rho_pd, const int *adj_off, const int *adj,
@@ -206,7 +207,7 @@ __global__ void __launch_bounds__(HT_THREADS, HT_WAVES) k_spmv_hex(
 // blocks are two loads a lane), a contiguous share of the rows per workgroup and, as in k_spmv_dot_p, of the
 // workgroups per XCD, one partial each, no second launch.  Bound by latency: 12 bytes per node pair, which
 // stay in the caches between the iterations, against the 76 of the 3D block walk.
-// 31^3 box (29,791 nodes, a PD block of 10^3): 8.0 us against 15.5 for the blocks and 4.0 for the fold.
+// 31^3 box (29,791 nodes, a PD block of 10^3): 8.0 us against 15.1 for the blocks and 4.3 for the fold.
 constexpr int MASS_THREADS = 1024;
 template <int D>
 __global__ void __launch_bounds__(MASS_THREADS) k_spmv_mass(int nn, const int *adj_off, const int *adj, const double *mass,

@@ -127,11 +127,13 @@ __global__ void __launch_bounds__(256) k_explicit(const int *rows_s, int ns, int
 // The same step without most of K: the rows of the nodes whose elements are all hex8 are formed from
 // the elements, those of the interior PD nodes from the moments of their families (hex.hpp), FP64 in
 // both precisions; the other rows (PD boundary and tetrahedron nodes) are walked in K, a wavefront
-// each, in the same launch.  On the 60^3 box (198,520 elements, 8,000 PD nodes) the step takes 44 us
-// where the best walk of K takes 75 in FP64 (80^3: 86 against 195, 100^3: 173 against 389), and 45 in
-// FP32: K is 330 MB (196 MB) per step there, while the elements are 8.6M FP64 wavefront instructions (15 us at the full rate) on some 60 MB.  Bound by
-// those two one after the other: two workgroups of 198 registers fit a CU, and the ones in flight load
-// together and calculate together.
+// each, in the same launch.  On the 60^3 box (198,520 elements, 8,000 PD nodes) the step takes 44 us in
+// replays of 120 steps, 47 on average under the tracer, where the best walk of K takes 76 in FP64 and 45
+// in FP32 (80^3: 82 against 186 and 120, 100^3: 139 against 361 and 240).  K is 330 MB (196 MB) per step
+// there; the tiles compute 326,864 elements, those between two tiles in both, in 11.5M vector
+// instructions (19 us at the full rate) and fetch 111 MB through the L2s.  Bound by those two one after
+// the other: two workgroups of 182 registers fit a CU, and the ones in flight load together and calculate
+// together (vector units busy 37% of the time, LDS 19%, a seventh of its cycles on bank conflicts).
 __global__ void __launch_bounds__(HT_THREADS, HT_WAVES) k_explicit_hex(
     HexTiles ht, MomentArgs ma, double lam8, double mu8, const int *adj_off, const int *adj, const double *K,
     const double *x, const double *Un, const double *Unm1, double *Unp1, const double *m, const double *f_unit, int n_nbc,
