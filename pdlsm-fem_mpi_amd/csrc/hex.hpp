@@ -83,7 +83,8 @@ inline double hex_walk_f32_us(double blocks) {
     return blocks <= 9e6 ? 7.0e-6 * blocks : 63.0 + 1.45e-5 * (blocks - 9e6);
 }
 // FP64 products go through the tiles up to this multiple of the walk's sum, FP32 products up to the walk's
-// own: on these models that is the faster way, or one within 3% of it.  FP64 steps through the tiles
+// own: on these models that is the faster way, or one within 3% of it (elsewhere the worst seen is 30^3 with
+// 8^3 PD nodes, 11.4 us through the tiles and 10.8 by the walk).  FP64 steps through the tiles
 // against the walk: 60^3 35 and 62 us, plate of 400 x 400 x 4 87 and 204, bar 5 x 5 x 8000 21 and 41; but
 // 300 x 300 x 2 52 and 38, 60^3 with a spacing of 1 : 10 70 and 62, of 1 : 100 148 and 62, with a fifth of
 // tetrahedra 95 and 59, a tenth of them spread out 216 and 62.  FP32: 80^3 72 and 113, 600 x 600 x 2 192
